@@ -86,18 +86,19 @@ hipError_t launch_mdf_weights(int nrows, int bsz, const int *rowpts, const doubl
                               double *Cw, hipStream_t s);
 hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
                                      int nlev, double *Mg, int *info, hipStream_t s);
-hipError_t launch_bilu0_lsolve_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, const double *Mg, const double *x, double *y, hipStream_t s);
-hipError_t launch_bilu0_usolve_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, const double *Mg, const double *y, double *v, hipStream_t s);
+// BILU0 sweeps: rows and nbr as RowSched (solver.hip), tickets [t0, t1) of one level
+hipError_t launch_bilu0_lsolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const double *Mg,
+                                     const double *x, double *y, hipStream_t s);
+hipError_t launch_bilu0_usolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const double *Mg,
+                                     const double *y, double *v, hipStream_t s);
 hipError_t launch_block_jacobi(int nrows, int bsz, const double *Dinv, const double *x, double *y, hipStream_t s);
 // single-precision preconditioner factors (FP32 storage, FP32 MFMA factorisation)
 hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
                                      int nlev, float *Mg, int *info, hipStream_t s);
-hipError_t launch_bilu0_lsolve_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, const float *Mg, const double *x, double *y, hipStream_t s);
-hipError_t launch_bilu0_usolve_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, const float *Mg, const double *y, double *v, hipStream_t s);
+hipError_t launch_bilu0_lsolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const float *Mg,
+                                     const double *x, double *y, hipStream_t s);
+hipError_t launch_bilu0_usolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const float *Mg,
+                                     const double *y, double *v, hipStream_t s);
 hipError_t launch_block_jacobi(int nrows, int bsz, const float *Dinv, const double *x, double *y, hipStream_t s);
 hipError_t launch_to_float(long n, const double *x, float *y, hipStream_t s);
 hipError_t launch_bilu0_factor_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o,
@@ -106,12 +107,12 @@ hipError_t launch_bilu0_factor_syncfree(int bsz, const int *rowpts, const int *c
 hipError_t launch_bilu0_factor_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o,
                                         const int *order, int n, float *Mg, int *info, unsigned *flags,
                                         unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s);
-hipError_t launch_bilu0_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *lorder,
-                                 const int *uorder, int n, const double *Mg, const double *x, double *t, double *y,
-                                 unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s);
-hipError_t launch_bilu0_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *lorder,
-                                 const int *uorder, int n, const float *Mg, const double *x, double *t, double *y,
-                                 unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s);
+hipError_t launch_bilu0_syncfree(int bsz, const int4 *lrows, const int2 *lnbr, const int4 *urows, const int2 *unbr,
+                                 int n, const double *Mg, const double *x, double *t, double *y, unsigned *sync,
+                                 int nwg, int spin_limit, int *err, hipStream_t s);
+hipError_t launch_bilu0_syncfree(int bsz, const int4 *lrows, const int2 *lnbr, const int4 *urows, const int2 *unbr,
+                                 int n, const float *Mg, const double *x, double *t, double *y, unsigned *sync,
+                                 int nwg, int spin_limit, int *err, hipStream_t s);
 int multidot_blocks(long n);
 hipError_t launch_multidot(long n, int k, const double *V, long ldv, const double *w, double *partial, double *out,
                            hipStream_t s);
@@ -145,7 +146,13 @@ struct SolverState {
     std::vector<int> o2u, u2o;          // host copies
     int *d_o2u = nullptr, *d_u2o = nullptr;
     std::vector<int> lptr, uptr;        // level pointers of the L (forward) and U (backward) sweeps
-    int *d_lrows = nullptr, *d_urows = nullptr;  // rows of each level, concatenated
+    std::vector<int> lrows, urows;      // rows of each level, concatenated
+    std::vector<int> llev, ulev;        // level of each row
+    bool sched_valid = false;           // the device copies below are the current ordering's
+    int *d_lrows = nullptr;             // lrows: the factorisation's order
+    // the sweeps' rows in level order with their neighbours (RowSched, solver.hip)
+    int4 *d_lsched = nullptr, *d_usched = nullptr;
+    int2 *d_lnbr = nullptr, *d_unbr = nullptr;
     double *Mg = nullptr;               // BILU0 factors (nblocks blocks) or block-Jacobi inverses (nf blocks)
     float *Mg32 = nullptr;              // the same in single precision (precPrecision 0)
     int prec_fp32 = 0;
@@ -155,9 +162,9 @@ struct SolverState {
     bool graph_dirty = true;
     int use_graph = 0;
     double *gy = nullptr;
-    // the BILU0 application without level launches (sweep_mode 1, default): 2 nf ready
-    // flags, then the epoch and two ticket counters; a flag set when a bounded wait
-    // gave up
+    // the BILU0 factorisation and application without level launches (sweep_mode 1,
+    // default): the factorisation's nf ready flags, then its epoch and the ticket
+    // counters; a flag set when a bounded wait gave up
     int sweep_mode = 1, spin_limit = 1 << 20, sweep_wgs = 1024;
     unsigned *sf_flags = nullptr;
     int *sf_err = nullptr;

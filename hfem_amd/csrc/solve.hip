@@ -100,18 +100,60 @@ static int build_levels(hfem_ctx *c)
             rows[fill[lev[r]]++] = r;
         }
     };
-    std::vector<int> lrows, urows;
-    bucket(lv, nl, s.lptr, lrows);
-    bucket(uv, nu, s.uptr, urows);
+    bucket(lv, nl, s.lptr, s.lrows);
+    bucket(uv, nu, s.uptr, s.urows);
+    s.llev = std::move(lv);
+    s.ulev = std::move(uv);
+    s.sched_valid = false;
+    s.prec = -2;                                       // factors belong to the previous ordering
+    return 0;
+}
+
+// The ordering and the schedules of the BILU0 kernels on the device, for the current
+// ordering (block-Jacobi needs none of them).
+static int ensure_schedule(hfem_ctx *c)
+{
+    SolverState &s = c->sv;
+    if (s.sched_valid) return 0;
+    const int n = c->hd.nf;
+    const std::vector<int> &rp = s.rowpts, &ci = s.colind;
+    // the sweeps' rows in level order, each with the neighbours it reads by increasing
+    // level (the last to be ready last)
+    auto schedule = [&](const std::vector<int> &rows, const std::vector<int> &lev, bool lower, std::vector<int4> &sched,
+                        std::vector<int2> &nbr) {
+        sched.resize(n);
+        nbr.clear();
+        nbr.reserve(ci.size() / 2 + 1);
+        for (int t = 0; t < n; t++) {
+            const int r = rows[t], first = (int)nbr.size();
+            for (int k = rp[r] + 1; k < rp[r + 1]; k++)
+                if ((s.u2o[ci[k]] < s.u2o[r]) == lower) nbr.push_back(make_int2(k, ci[k]));
+            std::sort(nbr.begin() + first, nbr.end(), [&](const int2 &a, const int2 &b) {
+                return lev[a.y] != lev[b.y] ? lev[a.y] < lev[b.y] : s.u2o[a.y] < s.u2o[b.y];
+            });
+            sched[t] = make_int4(r, rp[r], first, (int)nbr.size() - first);
+        }
+    };
+    std::vector<int4> lsched, usched;
+    std::vector<int2> lnbr, unbr;
+    schedule(s.lrows, s.llev, true, lsched, lnbr);
+    schedule(s.urows, s.ulev, false, usched, unbr);
     if (!s.d_lrows) HIPCHK(hfem_dalloc(&s.d_lrows, (size_t)n));
-    if (!s.d_urows) HIPCHK(hfem_dalloc(&s.d_urows, (size_t)n));
+    if (!s.d_lsched) HIPCHK(hfem_dalloc(&s.d_lsched, (size_t)n));
+    if (!s.d_usched) HIPCHK(hfem_dalloc(&s.d_usched, (size_t)n));
+    // (each holds at most every off-diagonal block)
+    if (!s.d_lnbr) HIPCHK(hfem_dalloc(&s.d_lnbr, ci.size()));
+    if (!s.d_unbr) HIPCHK(hfem_dalloc(&s.d_unbr, ci.size()));
     if (!s.d_o2u) HIPCHK(hfem_dalloc(&s.d_o2u, (size_t)n));
     if (!s.d_u2o) HIPCHK(hfem_dalloc(&s.d_u2o, (size_t)n));
-    HIPCHK(hipMemcpy(s.d_lrows, lrows.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(s.d_urows, urows.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(s.d_lrows, s.lrows.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(s.d_lsched, lsched.data(), sizeof(int4) * n, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(s.d_usched, usched.data(), sizeof(int4) * n, hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(s.d_lnbr, lnbr.data(), sizeof(int2) * lnbr.size(), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(s.d_unbr, unbr.data(), sizeof(int2) * unbr.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s.d_o2u, s.o2u.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s.d_u2o, s.u2o.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-    s.prec = -2;                                       // factors belong to the previous ordering
+    s.sched_valid = true;
     return 0;
 }
 
@@ -268,10 +310,11 @@ extern "C" int hfem_precond_factor(hfem_ctx *c, int kind)
         }
     } else {
         if (s.order_method < 0) RC(hfem_compute_ordering(c, 1));
+        RC(ensure_schedule(c));
         // (sync-free: one persistent launch over the rows in forward-level order;
         // else one launch per level)
         if (s.sweep_mode == 1) RC(ensure_syncfree(c));
-        unsigned *sync = s.sweep_mode == 1 ? s.sf_flags + 2 * (size_t)n : nullptr;
+        unsigned *sync = s.sweep_mode == 1 ? s.sf_flags + (size_t)n : nullptr;
         if (!fp32) {
             HIPCHK(hipMemcpyAsync(s.Mg, c->Hg, sizeof(double) * c->nblocks * b2, hipMemcpyDeviceToDevice, c->stream));
             if (s.sweep_mode == 1)
@@ -337,8 +380,8 @@ static int ensure_syncfree(hfem_ctx *c)
     if (s.lptr.empty() || s.lptr.back() != n || s.uptr.empty() || s.uptr.back() != n)
         return hfem_fail(-3, "sync-free BILU0 sweeps: the level lists do not cover the %d rows", n);
     if (!s.sf_flags) {
-        HIPCHK(hfem_dalloc(&s.sf_flags, (size_t)2 * n + 3));
-        HIPCHK(hipMemset(s.sf_flags, 0, sizeof(unsigned) * ((size_t)2 * n + 3)));
+        HIPCHK(hfem_dalloc(&s.sf_flags, (size_t)n + 3));
+        HIPCHK(hipMemset(s.sf_flags, 0, sizeof(unsigned) * ((size_t)n + 3)));
     }
     if (!s.sf_err) {
         HIPCHK(hfem_dalloc(&s.sf_err, 1));
@@ -370,27 +413,24 @@ static int bilu0_sweeps(hfem_ctx *c, const double *x, double *y)
     const int bsz = trace_bsz(c);
     if (s.sweep_mode == 1) {
         const int n = c->hd.nf;
+        unsigned *sync = s.sf_flags + (size_t)n;
         if (s.prec_fp32)
-            HIPCHK(launch_bilu0_syncfree(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lrows, s.d_urows, n, s.Mg32, x, s.t, y,
-                                         s.sf_flags, s.sf_flags + 2 * (size_t)n, s.sweep_wgs, s.spin_limit, s.sf_err,
-                                         c->stream));
+            HIPCHK(launch_bilu0_syncfree(bsz, s.d_lsched, s.d_lnbr, s.d_usched, s.d_unbr, n, s.Mg32, x, s.t, y, sync,
+                                         s.sweep_wgs, s.spin_limit, s.sf_err, c->stream));
         else
-            HIPCHK(launch_bilu0_syncfree(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lrows, s.d_urows, n, s.Mg, x, s.t, y,
-                                         s.sf_flags, s.sf_flags + 2 * (size_t)n, s.sweep_wgs, s.spin_limit, s.sf_err,
-                                         c->stream));
+            HIPCHK(launch_bilu0_syncfree(bsz, s.d_lsched, s.d_lnbr, s.d_usched, s.d_unbr, n, s.Mg, x, s.t, y, sync,
+                                         s.sweep_wgs, s.spin_limit, s.sf_err, c->stream));
         return 0;
     }
     for (size_t l = 0; l + 1 < s.lptr.size(); l++) {
-        const int *rows = s.d_lrows + s.lptr[l];
-        const int nl = s.lptr[l + 1] - s.lptr[l];
-        if (s.prec_fp32) HIPCHK(launch_bilu0_lsolve_level(bsz, c->rowstart, c->cols, s.d_u2o, rows, nl, s.Mg32, x, s.t, c->stream));
-        else HIPCHK(launch_bilu0_lsolve_level(bsz, c->rowstart, c->cols, s.d_u2o, rows, nl, s.Mg, x, s.t, c->stream));
+        const int t0 = s.lptr[l], t1 = s.lptr[l + 1];
+        if (s.prec_fp32) HIPCHK(launch_bilu0_lsolve_level(bsz, s.d_lsched, s.d_lnbr, t0, t1, s.Mg32, x, s.t, c->stream));
+        else HIPCHK(launch_bilu0_lsolve_level(bsz, s.d_lsched, s.d_lnbr, t0, t1, s.Mg, x, s.t, c->stream));
     }
     for (size_t l = 0; l + 1 < s.uptr.size(); l++) {
-        const int *rows = s.d_urows + s.uptr[l];
-        const int nl = s.uptr[l + 1] - s.uptr[l];
-        if (s.prec_fp32) HIPCHK(launch_bilu0_usolve_level(bsz, c->rowstart, c->cols, s.d_u2o, rows, nl, s.Mg32, s.t, y, c->stream));
-        else HIPCHK(launch_bilu0_usolve_level(bsz, c->rowstart, c->cols, s.d_u2o, rows, nl, s.Mg, s.t, y, c->stream));
+        const int t0 = s.uptr[l], t1 = s.uptr[l + 1];
+        if (s.prec_fp32) HIPCHK(launch_bilu0_usolve_level(bsz, s.d_usched, s.d_unbr, t0, t1, s.Mg32, s.t, y, c->stream));
+        else HIPCHK(launch_bilu0_usolve_level(bsz, s.d_usched, s.d_unbr, t0, t1, s.Mg, s.t, y, c->stream));
     }
     return 0;
 }

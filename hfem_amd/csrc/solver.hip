@@ -8,6 +8,7 @@
 #include "hfem_device.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace hfem {
 
@@ -483,122 +484,215 @@ __device__ __forceinline__ void wave_block_matvec(int bsz, const TM *__restrict_
     else wave_block_matvec_ch<64, false>(bsz, B, z0, z1, acc0, acc1);
 }
 
-// One BILU0 sweep over the rows of one level (kernel/applyBILU0.m).  For row r,
-// t = b_r - sum over the neighbours k taken by the sweep (numbered before r in the
-// forward sweep L y = x, after r in the backward sweep U v = y) of M_rk z_k; the
-// forward sweep stores z_r = t, the backward sweep z_r = inv(U_rr) t.  One
-// 256-thread workgroup per row: the four waves take the neighbour blocks in turn
-// (lane = block row, the neighbour vector broadcast from registers), their partial
-// sums meet in LDS.
-// The backward sweep's inv(U_rr) b_r, this wave's share: wave w takes the columns
-// cc = w, w + NW, ... of inv(U_rr) (preloaded in dv for blocks up to 64 wide, else
-// read from the block in chunks of 8 columns), b_r staged in LDS (tb); rows lane
-// (a0) and lane + 64 (a1).  Shared by both sweep kernels so that they compute the
-// same bits.
-template <bool SMALL, int ND, int NW, typename TM>
-__device__ __forceinline__ void inv_diag_share(int bsz, int wv, int lane, int r0, int r1, const TM *Ui,
-                                               const double (&dv)[ND], const double *tb, double &a0, double &a1)
+// ---- BILU0 sweeps (kernel/applyBILU0.m) ----
+//
+// For row r of a sweep, with neighbours k taken by it (numbered before r in the
+// forward sweep L y = x, after r in the backward sweep U v = y):
+//   forward   z_r = b_r - sum_k L_rk z_k
+//   backward  z_r = inv(U_rr) b_r - sum_k U~_rk z_k,  U~_rk = inv(U_rr) U_rk
+// (upper blocks scaled by the factorisation's last step, bilu0_scale_upper_kernel,
+// so that inv(U_rr) b_r is formed before the neighbours' z are needed).
+//
+// A sweep is bound by its chain of dependent rows (557 levels per sweep on 16 464
+// p=3 tets, 5 597 on 24^3 periodic p=2 hexes), so a row is laid out for the time
+// from its last neighbour's z to its own:
+// * One workgroup of four waves per row; every wave takes a quarter of the columns
+//   of every neighbour block (lane = block row), so what is left to do when the
+//   last z arrives is a quarter of one block product, one barrier and a sum of four.
+// * Blocks are loaded into registers before any wait, NPRE neighbours ahead.
+// * The neighbours come in the order of their level (RowSched, built with the
+//   levels), the last to be ready last.
+// * z itself is the ready flag: a sweep that runs as one launch fills z with a bit
+//   pattern no result has (SWEEP_EMPTY) and polls the entries it needs, so a hand-over is
+//   one store and one load (about 0.45 us between any two CUs; a separate flag behind
+//   a completed store, the earlier form, put three more round trips in each link).
+// Measured per application (two sweeps), FP64 factors, before with a flag per row and
+// one wave per whole block, and now:
+//   16 464 p=3 tets (block 50, 557 levels)         3.60 ms   1.82 ms
+//   8^3 periodic p=2 hexes (block 45, 370 levels)  2.68 ms   0.75 ms
+//   4 608 p=4 triangles (block 20, 849 levels)     4.82 ms   1.43 ms
+//   512 p=2 triangles (block 12, 104 levels)       0.63 ms   0.20 ms
+// i.e. 0.85-1.0 us per link; the large mesh is bound by reading its factors (4.6 GB)
+// next to the chain.
+struct RowSched {
+    const int4 *rows;    // by ticket: row, its diagonal block, first entry in nbr, neighbours
+    const int2 *nbr;     // block, column
+};
+
+// A signalling NaN: stored results are quieted, never equal to it.
+constexpr unsigned long long SWEEP_EMPTY = 0x7ff4dead5eed0001ull;
+
+// Until lane's *p is no longer SWEEP_EMPTY in any lane: its value.  Entries are read
+// and written by agent-scope atomics (coherent across the XCDs).  At most spin_limit
+// polls after the first; a wait that runs out, or any wait once another has (*err
+// set), sets *err and returns.
+__device__ __forceinline__ double wait_entry(const double *p, int spin_limit, int *err)
 {
-    a0 = 0.0;
-    a1 = 0.0;
-    if (SMALL) {
-#pragma unroll
-        for (int j = 0; j < ND; j++) {
-            const int cc = wv + NW * j;
-            a0 += dv[j] * (cc < bsz ? tb[min(cc, bsz - 1)] : 0.0);
+    unsigned long long v;
+    int spins = 0;
+    // (the ballot makes the loop's control wave-uniform)
+    while (true) {
+        v = __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (__ballot(v == SWEEP_EMPTY) == 0) break;
+        if (++spins > spin_limit ||
+            ((spins & 63) == 0 && __builtin_amdgcn_readfirstlane(
+                                      __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))) {
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            break;
         }
-    } else {
-        // (loads of 8 columns issued together, addresses clamped into the block)
-        for (int c0 = wv; c0 < bsz; c0 += 8 * NW) {
-            double v0[8], v1[8];
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const long col = (long)bsz * min(c0 + j * NW, bsz - 1);
-                v0[j] = Ui[r0 + col];
-                v1[j] = Ui[r1 + col];
-            }
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                const int cc = c0 + j * NW;
-                const double tc = cc < bsz ? tb[min(cc, bsz - 1)] : 0.0;
-                a0 += v0[j] * tc;
-                a1 += v1[j] * tc;
-            }
-        }
+        __builtin_amdgcn_s_sleep(1);
     }
-    if (lane >= bsz) a0 = 0.0;
-    if (lane + 64 >= bsz) a1 = 0.0;
+    return __longlong_as_double((long long)v);
 }
 
-// Backward sweeps read upper blocks scaled by the factorisation's last step
-// (bilu0_scale_upper_kernel): U~_rl = inv(U_rr) U_rl, so that
-//   z_r = inv(U_rr) b_r - sum_l U~_rl z_l
-// and inv(U_rr) b_r is formed before the neighbours' z are needed.
-template <bool BACKWARD, bool SMALL, typename TM>
-__global__ void __launch_bounds__(SV_THREADS)
-bilu0_sweep_kernel(int bsz, const int *__restrict__ rowpts, const int *__restrict__ colind,
-                   const int *__restrict__ u2o, const int *__restrict__ rows, int nlev, const TM *__restrict__ Mg,
-                   const double *__restrict__ b, double *__restrict__ z)
+// One row of a sweep, the ticket t's, by the whole workgroup.  The lane holds block
+// rows lane (+ 64 with RCH 2); wave w the columns [w cpw, (w+1) cpw) of each block,
+// cpw = ceil(bsz / 4) <= CPW.  Loads are clamped into the block and columns past the
+// wave's multiplied by zero.  Shared by the one-launch (WAIT) and level-launched
+// kernels so that both compute the same bits.
+template <bool BACKWARD, int RCH, int CPW, int NPRE, bool WAIT, typename TM>
+__device__ __forceinline__ void sweep_row(int bsz, const RowSched &sch, int t, const TM *__restrict__ Mg,
+                                          const double *__restrict__ b, double *z, double (*red)[64 * RCH],
+                                          int spin_limit, int *err)
 {
     constexpr int NW = SV_THREADS / 64;
-    __shared__ double red[NW][128];
-    __shared__ double tb[128];
-    __shared__ int scol[FACTOR_MAXROW], stake[FACTOR_MAXROW];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const long b2 = (long)bsz * bsz;
-    const int r0 = lane < bsz ? lane : 0, r1 = lane + 64 < bsz ? lane + 64 : 0;
-    for (int t = blockIdx.x; t < nlev; t += gridDim.x) {
-        const int r = rows[t], o = u2o[r], k0 = rowpts[r], len = min(rowpts[r + 1] - k0, FACTOR_MAXROW);
-        const TM *Ui = Mg + (long)k0 * b2;
-        // the loads that depend on nothing else go out together: the row's column
-        // list (rows have at most FACTOR_MAXROW blocks: the factorisation rejects
-        // longer ones), its right-hand side and, backward, this wave's columns
-        // wv + NW j of inv(U_rr)
-        if (tid < len) {
-            const int c = colind[k0 + tid];
-            scol[tid] = c;
-            stake[tid] = BACKWARD ? (u2o[c] > o) : (u2o[c] < o);
-        }
-        const double bv = tid < bsz ? b[(long)r * bsz + tid] : 0.0;
-        if (BACKWARD && tid < bsz) tb[tid] = bv;
-        constexpr int ND = (SMALL && BACKWARD) ? 64 / NW : 1;
-        double dv[ND];
-        if (SMALL && BACKWARD) {
+    const int cpw = (bsz + NW - 1) / NW, c0 = wv * cpw;
+    const int4 h = sch.rows[t];
+    const int r = __builtin_amdgcn_readfirstlane(h.x), kd = __builtin_amdgcn_readfirstlane(h.y);
+    const int first = __builtin_amdgcn_readfirstlane(h.z), cnt = __builtin_amdgcn_readfirstlane(h.w);
+    const int2 *nbr = sch.nbr + first;
+    int rl[RCH];
 #pragma unroll
-            for (int j = 0; j < ND; j++) dv[j] = Ui[r0 + (long)bsz * min(wv + NW * j, bsz - 1)];
-        }
-        __syncthreads();
-        double p0 = 0.0, p1 = 0.0;
-        if (BACKWARD) inv_diag_share<SMALL, ND, NW>(bsz, wv, lane, r0, r1, Ui, dv, tb, p0, p1);
-        double acc0 = 0.0, acc1 = 0.0;
-        int sel = 0;
-        for (int q = 1; q < len; q++) {
-            if (!stake[q]) continue;
-            if ((sel++ % NW) != wv) continue;
-            const int c = scol[q];
-            const double *zc = z + (long)c * bsz;
-            const double z0 = lane < bsz ? zc[lane] : 0.0, z1 = lane + 64 < bsz ? zc[lane + 64] : 0.0;
-            if (SMALL) wave_block_matvec_ch<64, false>(bsz, Mg + (long)(k0 + q) * b2, z0, z1, acc0, acc1);
-            else wave_block_matvec_ch<16, true>(bsz, Mg + (long)(k0 + q) * b2, z0, z1, acc0, acc1);
-        }
-        red[wv][lane] = BACKWARD ? p0 - acc0 : acc0;
-        red[wv][lane + 64] = BACKWARD ? p1 - acc1 : acc1;
-        __syncthreads();
-        if (tid < bsz) {
-            double sum = 0.0;
+    for (int q = 0; q < RCH; q++) rl[q] = min(lane + 64 * q, bsz - 1);
+    const int ce = min(c0 + min(lane, cpw - 1), bsz - 1);       // the vector entry this lane fetches
+    const bool cv = lane < cpw && c0 + lane < bsz;
+    auto load_share = [&](int blk, TM (&v)[CPW][RCH]) {
+        const TM *B = Mg + (long)blk * b2;
 #pragma unroll
-            for (int w = 0; w < NW; w++) sum += red[w][tid];
-            z[(long)r * bsz + tid] = BACKWARD ? sum : bv - sum;
+        for (int j = 0; j < CPW; j++)
+#pragma unroll
+            for (int q = 0; q < RCH; q++) v[j][q] = B[rl[q] + (long)bsz * min(c0 + j, bsz - 1)];
+    };
+    auto add_share = [&](const TM (&v)[CPW][RCH], double ze, double (&acc)[RCH]) {
+        const double zm = cv ? ze : 0.0;
+#pragma unroll
+        for (int j = 0; j < CPW; j++) {
+            const double zj = wave_bcast(zm, j);
+#pragma unroll
+            for (int q = 0; q < RCH; q++) acc[q] += (double)v[j][q] * zj;
         }
+    };
+    TM v[NPRE][CPW][RCH];
+#pragma unroll
+    for (int i = 0; i < NPRE; i++)
+        if (i < cnt) load_share(__builtin_amdgcn_readfirstlane(nbr[i].x), v[i]);
+    double own[RCH], acc[RCH];
+#pragma unroll
+    for (int q = 0; q < RCH; q++) {
+        own[q] = 0.0;
+        acc[q] = 0.0;
+    }
+    if (BACKWARD) {
+        TM dv[CPW][RCH];
+        load_share(kd, dv);
+        add_share(dv, b[(long)r * bsz + ce], own);
+    } else if (wv == 0) {
+#pragma unroll
+        for (int q = 0; q < RCH; q++) own[q] = b[(long)r * bsz + rl[q]];
+    }
+    for (int i0 = 0; i0 < cnt; i0 += NPRE) {
+#pragma unroll
+        for (int i = 0; i < NPRE; i++) {
+            if (i0 + i >= cnt) break;
+            const double *ze = z + (long)__builtin_amdgcn_readfirstlane(nbr[i0 + i].y) * bsz + ce;
+            add_share(v[i], WAIT ? wait_entry(ze, spin_limit, err) : *ze, acc);
+            if (i0 + NPRE + i < cnt) load_share(__builtin_amdgcn_readfirstlane(nbr[i0 + NPRE + i].x), v[i]);
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < RCH; q++) red[wv][lane + 64 * q] = own[q] - acc[q];
+    __syncthreads();
+    if (wv == 0) {
+#pragma unroll
+        for (int q = 0; q < RCH; q++) {
+            double s = red[0][lane + 64 * q];
+#pragma unroll
+            for (int w = 1; w < NW; w++) s += red[w][lane + 64 * q];
+            unsigned long long u = (unsigned long long)__double_as_longlong(s);
+            u = u == SWEEP_EMPTY ? 0x7ff8000000000000ull : u;
+            double *zr = z + (long)r * bsz + lane + 64 * q;
+            if (lane + 64 * q < bsz) {
+                if (WAIT) __hip_atomic_store((unsigned long long *)zr, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                else *zr = __longlong_as_double((long long)u);
+            }
+        }
+    }
+}
+
+// The rows of one level: tickets [t0, t1).
+template <bool BACKWARD, int RCH, int CPW, int NPRE, typename TM>
+__global__ void __launch_bounds__(SV_THREADS)
+bilu0_sweep_kernel(int bsz, RowSched sch, int t0, int t1, const TM *__restrict__ Mg, const double *__restrict__ b,
+                   double *z)
+{
+    __shared__ double red[SV_THREADS / 64][64 * RCH];
+    for (int t = t0 + blockIdx.x; t < t1; t += gridDim.x) {
+        sweep_row<BACKWARD, RCH, CPW, NPRE, false, TM>(bsz, sch, t, Mg, b, z, red, 0, nullptr);
         __syncthreads();
     }
 }
 
-// Wait until *f holds `epoch`.  The flags and the vector entries they guard are
-// read and written only by agent-scope atomics (coherent across the XCDs without
-// whole-L2 write-backs or invalidations, which an acquire / release pair costs
-// here per row).  At most spin_limit polls; a wait that runs out, or any wait once
-// another has (*err set), sets *err and returns.
+// A whole sweep in one launch: the rows in ticket order -- the level lists
+// concatenated, so every row comes after the rows it reads -- to persistent
+// workgroups through an atomic ticket.  A wait that gives up (wait_entry) leaves a
+// wrong result and *err set, which the host reports; every workgroup still runs to
+// the end of the tickets.  No deadlock: a workgroup waits only on rows of smaller
+// tickets, which were drawn by workgroups already running.
+template <bool BACKWARD, int RCH, int CPW, int NPRE, typename TM>
+__global__ void __launch_bounds__(SV_THREADS)
+bilu0_sweep_syncfree_kernel(int bsz, RowSched sch, int n, const TM *__restrict__ Mg, const double *__restrict__ b,
+                            double *z, unsigned *counter, int spin_limit, int *err)
+{
+    __shared__ double red[SV_THREADS / 64][64 * RCH];
+    __shared__ int sticket;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // The ticket is drawn by the whole of wave 0 (a wave-uniform condition): the draw
+    // adds 1 from lane 0 and 0 from the others, and lane 0's old value is the ticket.
+    // Under "tid == 0" the structurizer may merge the draw across the back edge into
+    // an inner loop that only lane 0 leaves.
+    while (true) {
+        if (wv == 0) sticket = __builtin_amdgcn_readfirstlane(atomicAdd(counter, lane == 0 ? 1u : 0u));
+        // (also: wave 0 has summed the previous row's red before any wave writes it again)
+        __syncthreads();
+        const int t = __builtin_amdgcn_readfirstlane(sticket);
+        if (t >= n) break;
+        sweep_row<BACKWARD, RCH, CPW, NPRE, true, TM>(bsz, sch, t, Mg, b, z, red, spin_limit, err);
+    }
+}
+
+// Fresh tickets for the two sweeps of an application and their empty results (a
+// kernel, not a memset, so that the application can be captured in a graph).
+__global__ void __launch_bounds__(SV_THREADS)
+sweep_reset_kernel(unsigned *sync, long n, double *t, double *y)
+{
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        sync[1] = 0;
+        sync[2] = 0;
+    }
+    const double e = __longlong_as_double((long long)SWEEP_EMPTY);
+    for (long i = blockIdx.x * (long)blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) {
+        t[i] = e;
+        y[i] = e;
+    }
+}
+
+// Wait until *f holds `epoch`, for the factorisation's ready flags.  The flags and
+// the blocks they guard are read and written only by agent-scope atomics (coherent
+// across the XCDs without whole-L2 write-backs or invalidations, which an acquire /
+// release pair costs here per row).  At most spin_limit polls; a wait that runs out,
+// or any wait once another has (*err set), sets *err and returns.
 __device__ __forceinline__ void wait_ready(const unsigned *f, unsigned epoch, int spin_limit, int *err)
 {
     // (the polled values go through readfirstlane: a uniform loop)
@@ -614,130 +708,6 @@ __device__ __forceinline__ void wait_ready(const unsigned *f, unsigned epoch, in
     }
 }
 
-// One BILU0 sweep without level launches (kernel/applyBILU0.m), with the per-row
-// arithmetic of bilu0_sweep_kernel (the same bits).  The rows go in `order` -- the
-// level lists concatenated, so every row comes after the rows it reads -- to
-// persistent workgroups through an atomic ticket.  A wave issues the loads of a
-// neighbour block (bsz <= 64: all 64 columns into registers) before it waits for
-// that neighbour's ready flag, so the block's latency overlaps the wait.  Vector
-// entries written in the sweep are stored and read by agent-scope atomics; the row's
-// flag is stored once those stores have completed (workgroup fence, then barrier).
-// Flags hold the
-// epoch of the current application (sweep_reset_kernel bumps it), so they are never
-// cleared.  A wait that gives up (wait_ready) leaves a wrong result and *err set,
-// which the host reports; every workgroup still runs to the end of the tickets.
-// No deadlock: a workgroup waits only on rows of smaller tickets, which were drawn
-// by workgroups already running.
-template <bool BACKWARD, bool SMALL, typename TM>
-__global__ void __launch_bounds__(SV_THREADS)
-bilu0_sweep_syncfree_kernel(int bsz, const int *__restrict__ rowpts, const int *__restrict__ colind,
-                            const int *__restrict__ u2o, const int *__restrict__ order, int n,
-                            const TM *__restrict__ Mg, const double *__restrict__ b, double *z, unsigned *flags,
-                            const unsigned *epoch_p, unsigned *counter, int spin_limit, int *err)
-{
-    constexpr int NW = SV_THREADS / 64;
-    __shared__ double red[NW][128];
-    __shared__ double tb[128];
-    __shared__ int scol[FACTOR_MAXROW], stake[FACTOR_MAXROW];
-    __shared__ int sticket;
-    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const long b2 = (long)bsz * bsz;
-    const int r0 = lane < bsz ? lane : 0, r1 = lane + 64 < bsz ? lane + 64 : 0;
-    const unsigned epoch = __hip_atomic_load(epoch_p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // No lane-conditional code may sit between the last barrier of one row and the
-    // first of the next: with the flag store and the ticket draw both under
-    // "tid == 0", the structurizer merged them across the back edge into an inner
-    // loop that only lane 0 leaves, so the other lanes re-ran the old row forever.
-    // Both are therefore done by the whole of wave 0 (a wave-uniform condition):
-    // the draw adds 1 from lane 0 and 0 from the others, and lane 0's old value is
-    // the ticket; every lane stores the same flag.
-    while (true) {
-        if (wv == 0) sticket = __builtin_amdgcn_readfirstlane(atomicAdd(counter, lane == 0 ? 1u : 0u));
-        __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(sticket);
-        if (t >= n) break;
-        const int r = order[t], o = u2o[r], k0 = rowpts[r], len = min(rowpts[r + 1] - k0, FACTOR_MAXROW);
-        const TM *Ui = Mg + (long)k0 * b2;
-        if (tid < len) {
-            const int c = colind[k0 + tid];
-            scol[tid] = c;
-            stake[tid] = BACKWARD ? (u2o[c] > o) : (u2o[c] < o);
-        }
-        // the right-hand side of entries lane and lane + 64, for wave 0, which
-        // stores the row (so that its own wait covers every store of the row)
-        const double bv0 = wv == 0 && lane < bsz ? b[(long)r * bsz + lane] : 0.0;
-        const double bv1 = wv == 0 && lane + 64 < bsz ? b[(long)r * bsz + lane + 64] : 0.0;
-        if (BACKWARD && tid < bsz) tb[tid] = b[(long)r * bsz + tid];
-        constexpr int ND = (SMALL && BACKWARD) ? 64 / NW : 1;
-        double dv[ND];
-        if (SMALL && BACKWARD) {
-#pragma unroll
-            for (int j = 0; j < ND; j++) dv[j] = Ui[r0 + (long)bsz * min(wv + NW * j, bsz - 1)];
-        }
-        __syncthreads();
-        // backward: inv(U_rr) b_r before any wait on a neighbour
-        double p0 = 0.0, p1 = 0.0;
-        if (BACKWARD) inv_diag_share<SMALL, ND, NW>(bsz, wv, lane, r0, r1, Ui, dv, tb, p0, p1);
-        double acc0 = 0.0, acc1 = 0.0;
-        int sel = 0;
-        for (int q = 1; q < len; q++) {
-            if (!__builtin_amdgcn_readfirstlane(stake[q])) continue;
-            if ((sel++ % NW) != wv) continue;
-            const int c = __builtin_amdgcn_readfirstlane(scol[q]);
-            const TM *B = Mg + (long)(k0 + q) * b2;
-            const double *zc = z + (long)c * bsz;
-            if (SMALL) {
-                double v0[64];
-#pragma unroll
-                for (int j = 0; j < 64; j++) v0[j] = B[r0 + (long)bsz * min(j, bsz - 1)];
-                wait_ready(flags + c, epoch, spin_limit, err);
-                const double z0 = lane < bsz ? __hip_atomic_load(zc + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                             : 0.0;
-                double s0 = 0.0;
-#pragma unroll
-                for (int j = 0; j < 64; j++) {
-                    double zj = wave_bcast(z0, j);
-                    zj = j < bsz ? zj : 0.0;
-                    s0 += v0[j] * zj;
-                }
-                if (lane < bsz) acc0 += s0;
-            } else {
-                wait_ready(flags + c, epoch, spin_limit, err);
-                const double z0 =
-                    lane < bsz ? __hip_atomic_load(zc + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0.0;
-                const double z1 =
-                    lane + 64 < bsz ? __hip_atomic_load(zc + lane + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                    : 0.0;
-                wave_block_matvec_ch<16, true>(bsz, B, z0, z1, acc0, acc1);
-            }
-        }
-        red[wv][lane] = BACKWARD ? p0 - acc0 : acc0;
-        red[wv][lane + 64] = BACKWARD ? p1 - acc1 : acc1;
-        __syncthreads();
-        if (wv == 0) {
-#pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const int i = lane + 64 * h;
-                if (i < bsz) {
-                    double sum = 0.0;
-#pragma unroll
-                    for (int w = 0; w < NW; w++) sum += red[w][i];
-                    const double v = BACKWARD ? sum : (h ? bv1 : bv0) - sum;
-                    __hip_atomic_store(z + (long)r * bsz + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
-        }
-        // publish row r: wave 0 stored it; once its stores have completed (vmcnt 0:
-        // device-scope stores are acknowledged at the coherence point) the flag goes
-        // out.  (The barrier also frees red, tb and the column lists for the next row.)
-        if (wv == 0) __builtin_amdgcn_s_waitcnt(0x0F70);   // s_waitcnt vmcnt(0)
-        __syncthreads();
-        if (wv == 0) __hip_atomic_store(flags + r, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-// A new epoch for the flags of the next application and fresh tickets for its two
-// sweeps (a kernel, not a memset, so that the application can be captured in a graph).
 // The factorisation's last step for the sweeps: every upper block of row r becomes
 // U~_rl = inv(U_rr) U_rl (inv(U_rr) is the row's diagonal block), in place, after
 // the whole factorisation (the other rows' eliminations read the unscaled U_rl).
@@ -780,13 +750,14 @@ bilu0_scale_upper_kernel(int bsz, int n, const int *__restrict__ rowpts, const i
     }
 }
 
-__global__ void sweep_reset_kernel(unsigned *sync)
+// A new epoch for the factorisation's ready flags (so that they are never cleared)
+// and a fresh ticket.
+__global__ void factor_reset_kernel(unsigned *sync)
 {
     if (threadIdx.x == 0) {
         unsigned e = sync[0] + 1;
         sync[0] = e == 0 ? 1 : e;
         sync[1] = 0;
-        sync[2] = 0;
     }
 }
 
@@ -1121,7 +1092,7 @@ static hipError_t factor_syncfree(int bsz, const int *rowpts, const int *colind,
     const size_t lds = bilu0_factor_lds(bsz) + 16;   // and the ticket
     hipError_t e = set_lds((const void *)bilu0_factor_syncfree_kernel<T>, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(sweep_reset_kernel, dim3(1), dim3(64), 0, s, sync);
+    hipLaunchKernelGGL(factor_reset_kernel, dim3(1), dim3(64), 0, s, sync);
     hipLaunchKernelGGL(bilu0_factor_syncfree_kernel<T>, dim3(std::min(n, nwg)), dim3(SV_THREADS), lds, s, bsz, rowpts,
                        colind, u2o, order, n, Mg, info, flags, sync, sync + 1, spin_limit, err);
     return hipGetLastError();
@@ -1175,78 +1146,92 @@ hipError_t launch_bilu0_scale_upper(int bsz, int n, const int *rowpts, const int
     return scale_upper(bsz, n, rowpts, colind, u2o, Mg, s);
 }
 
+// The sweep kernels' shapes by block size: CPW columns per wave, NPRE neighbours'
+// shares in registers (up to about 128 VGPRs of them).  A shape's unused columns cost
+// their loads, so the sizes in use have one that fits: 8-16 (triangles p=1-3), 20 and
+// 24 (p=4, 5, hexes p=1), 30 (tets p=2), 45 (hexes p=2), 50 (tets p=3); 75 (tets p=4)
+// and above take two rows per lane.
+template <class F>
+static hipError_t sweep_shape(int bsz, F launch)
+{
+    using std::integral_constant;
+#define SHAPE(R, C, P) \
+    launch(integral_constant<int, R>(), integral_constant<int, C>(), integral_constant<int, P>())
+    if (bsz < 1 || bsz > 128) return hipErrorInvalidValue;
+    if (bsz <= 16) SHAPE(1, 4, 8);
+    else if (bsz <= 24) SHAPE(1, 6, 8);
+    else if (bsz <= 32) SHAPE(1, 8, 6);
+    else if (bsz <= 48) SHAPE(1, 12, 5);
+    else if (bsz <= 52) SHAPE(1, 13, 4);
+    else if (bsz <= 64) SHAPE(1, 16, 4);
+    else if (bsz <= 80) SHAPE(2, 20, 1);
+    else SHAPE(2, 32, 1);
+#undef SHAPE
+    return hipGetLastError();
+}
+
 template <bool BACKWARD, typename TM>
-static hipError_t sweep_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                              int nlev, const TM *Mg, const double *x, double *y, hipStream_t s)
+static hipError_t sweep_level(int bsz, const RowSched &sch, int t0, int t1, const TM *Mg, const double *x, double *y,
+                              hipStream_t s)
 {
-    if (bsz > 128) return hipErrorInvalidValue;
-    if (bsz <= 64)
-        hipLaunchKernelGGL((bilu0_sweep_kernel<BACKWARD, true, TM>), dim3(std::min(nlev, 8192)), dim3(SV_THREADS), 0,
-                           s, bsz, rowpts, colind, u2o, rows, nlev, Mg, x, y);
-    else
-        hipLaunchKernelGGL((bilu0_sweep_kernel<BACKWARD, false, TM>), dim3(std::min(nlev, 8192)), dim3(SV_THREADS), 0,
-                           s, bsz, rowpts, colind, u2o, rows, nlev, Mg, x, y);
-    return hipGetLastError();
+    return sweep_shape(bsz, [&](auto R, auto C, auto P) {
+        hipLaunchKernelGGL((bilu0_sweep_kernel<BACKWARD, R(), C(), P(), TM>), dim3(std::min(t1 - t0, 8192)),
+                           dim3(SV_THREADS), 0, s, bsz, sch, t0, t1, Mg, x, y);
+    });
 }
 
-hipError_t launch_bilu0_lsolve_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, const double *Mg, const double *x, double *y, hipStream_t s)
+hipError_t launch_bilu0_lsolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const double *Mg,
+                                     const double *x, double *y, hipStream_t s)
 {
-    return sweep_level<false>(bsz, rowpts, colind, u2o, rows, nlev, Mg, x, y, s);
+    return sweep_level<false>(bsz, RowSched{rows, nbr}, t0, t1, Mg, x, y, s);
 }
-hipError_t launch_bilu0_lsolve_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, const float *Mg, const double *x, double *y, hipStream_t s)
+hipError_t launch_bilu0_lsolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const float *Mg,
+                                     const double *x, double *y, hipStream_t s)
 {
-    return sweep_level<false>(bsz, rowpts, colind, u2o, rows, nlev, Mg, x, y, s);
+    return sweep_level<false>(bsz, RowSched{rows, nbr}, t0, t1, Mg, x, y, s);
 }
-hipError_t launch_bilu0_usolve_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, const double *Mg, const double *y, double *v, hipStream_t s)
+hipError_t launch_bilu0_usolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const double *Mg,
+                                     const double *y, double *v, hipStream_t s)
 {
-    return sweep_level<true>(bsz, rowpts, colind, u2o, rows, nlev, Mg, y, v, s);
+    return sweep_level<true>(bsz, RowSched{rows, nbr}, t0, t1, Mg, y, v, s);
 }
-hipError_t launch_bilu0_usolve_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, const float *Mg, const double *y, double *v, hipStream_t s)
+hipError_t launch_bilu0_usolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const float *Mg,
+                                     const double *y, double *v, hipStream_t s)
 {
-    return sweep_level<true>(bsz, rowpts, colind, u2o, rows, nlev, Mg, y, v, s);
+    return sweep_level<true>(bsz, RowSched{rows, nbr}, t0, t1, Mg, y, v, s);
 }
 
-// Both sweeps of one BILU0 application without level launches: x -> t (forward,
-// rows in lorder) -> y (backward, rows in uorder).  sync: [0] epoch, [1], [2] the
-// tickets of the two sweeps; flags: n forward then n backward ready flags.
+// Both sweeps of one BILU0 application without level launches: x -> t (forward) ->
+// y (backward).  sync: [1], [2] the tickets of the two sweeps.
 template <typename TM>
-static hipError_t sweeps_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *lorder,
-                                  const int *uorder, int n, const TM *Mg, const double *x, double *t, double *y,
-                                  unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s)
+static hipError_t sweeps_syncfree(int bsz, const RowSched &low, const RowSched &up, int n, const TM *Mg, const double *x,
+                                  double *t, double *y, unsigned *sync, int nwg, int spin_limit, int *err,
+                                  hipStream_t s)
 {
-    if (bsz > 128 || n <= 0 || nwg <= 0) return hipErrorInvalidValue;
+    if (n <= 0 || nwg <= 0) return hipErrorInvalidValue;
     const int g = std::min(n, nwg);
-    hipLaunchKernelGGL(sweep_reset_kernel, dim3(1), dim3(64), 0, s, sync);
-    if (bsz <= 64) {
-        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<false, true, TM>), dim3(g), dim3(SV_THREADS), 0, s, bsz, rowpts,
-                           colind, u2o, lorder, n, Mg, x, t, flags, sync, sync + 1, spin_limit, err);
-        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<true, true, TM>), dim3(g), dim3(SV_THREADS), 0, s, bsz, rowpts,
-                           colind, u2o, uorder, n, Mg, t, y, flags + n, sync, sync + 2, spin_limit, err);
-    } else {
-        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<false, false, TM>), dim3(g), dim3(SV_THREADS), 0, s, bsz,
-                           rowpts, colind, u2o, lorder, n, Mg, x, t, flags, sync, sync + 1, spin_limit, err);
-        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<true, false, TM>), dim3(g), dim3(SV_THREADS), 0, s, bsz,
-                           rowpts, colind, u2o, uorder, n, Mg, t, y, flags + n, sync, sync + 2, spin_limit, err);
-    }
-    return hipGetLastError();
+    const long N = (long)n * bsz;
+    hipLaunchKernelGGL(sweep_reset_kernel, dim3(grid_for(N)), dim3(SV_THREADS), 0, s, sync, N, t, y);
+    return sweep_shape(bsz, [&](auto R, auto C, auto P) {
+        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<false, R(), C(), P(), TM>), dim3(g), dim3(SV_THREADS), 0, s,
+                           bsz, low, n, Mg, x, t, sync + 1, spin_limit, err);
+        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<true, R(), C(), P(), TM>), dim3(g), dim3(SV_THREADS), 0, s,
+                           bsz, up, n, Mg, t, y, sync + 2, spin_limit, err);
+    });
 }
 
-hipError_t launch_bilu0_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *lorder,
-                                 const int *uorder, int n, const double *Mg, const double *x, double *t, double *y,
-                                 unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s)
+hipError_t launch_bilu0_syncfree(int bsz, const int4 *lrows, const int2 *lnbr, const int4 *urows, const int2 *unbr,
+                                 int n, const double *Mg, const double *x, double *t, double *y, unsigned *sync,
+                                 int nwg, int spin_limit, int *err, hipStream_t s)
 {
-    return sweeps_syncfree(bsz, rowpts, colind, u2o, lorder, uorder, n, Mg, x, t, y, flags, sync, nwg, spin_limit,
+    return sweeps_syncfree(bsz, RowSched{lrows, lnbr}, RowSched{urows, unbr}, n, Mg, x, t, y, sync, nwg, spin_limit,
                            err, s);
 }
-hipError_t launch_bilu0_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *lorder,
-                                 const int *uorder, int n, const float *Mg, const double *x, double *t, double *y,
-                                 unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s)
+hipError_t launch_bilu0_syncfree(int bsz, const int4 *lrows, const int2 *lnbr, const int4 *urows, const int2 *unbr,
+                                 int n, const float *Mg, const double *x, double *t, double *y, unsigned *sync,
+                                 int nwg, int spin_limit, int *err, hipStream_t s)
 {
-    return sweeps_syncfree(bsz, rowpts, colind, u2o, lorder, uorder, n, Mg, x, t, y, flags, sync, nwg, spin_limit,
+    return sweeps_syncfree(bsz, RowSched{lrows, lnbr}, RowSched{urows, unbr}, n, Mg, x, t, y, sync, nwg, spin_limit,
                            err, s);
 }
 
