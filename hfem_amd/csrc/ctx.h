@@ -84,8 +84,8 @@ hipError_t launch_block_inverse(int nrows, int bsz, const int *rowpts, const dou
                                 hipStream_t s);
 hipError_t launch_mdf_weights(int nrows, int bsz, const int *rowpts, const double *Hg, const double *Dinv,
                               double *Cw, hipStream_t s);
-hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, double *Mg, int *info, hipStream_t s);
+hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int4 *rows,
+                                     const int2 *nbr, int t0, int t1, double *Mg, int *info, hipStream_t s);
 // BILU0 sweeps: rows and nbr as RowSched (solver.hip), tickets [t0, t1) of one level
 hipError_t launch_bilu0_lsolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const double *Mg,
                                      const double *x, double *y, hipStream_t s);
@@ -93,8 +93,8 @@ hipError_t launch_bilu0_usolve_level(int bsz, const int4 *rows, const int2 *nbr,
                                      const double *y, double *v, hipStream_t s);
 hipError_t launch_block_jacobi(int nrows, int bsz, const double *Dinv, const double *x, double *y, hipStream_t s);
 // single-precision preconditioner factors (FP32 storage, FP32 MFMA factorisation)
-hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, float *Mg, int *info, hipStream_t s);
+hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int4 *rows,
+                                     const int2 *nbr, int t0, int t1, float *Mg, int *info, hipStream_t s);
 hipError_t launch_bilu0_lsolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const float *Mg,
                                      const double *x, double *y, hipStream_t s);
 hipError_t launch_bilu0_usolve_level(int bsz, const int4 *rows, const int2 *nbr, int t0, int t1, const float *Mg,
@@ -102,11 +102,13 @@ hipError_t launch_bilu0_usolve_level(int bsz, const int4 *rows, const int2 *nbr,
 hipError_t launch_block_jacobi(int nrows, int bsz, const float *Dinv, const double *x, double *y, hipStream_t s);
 hipError_t launch_to_float(long n, const double *x, float *y, hipStream_t s);
 hipError_t launch_bilu0_factor_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o,
-                                        const int *order, int n, double *Mg, int *info, unsigned *flags,
-                                        unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s);
+                                        const int4 *rows, const int2 *nbr, int n, double *Mg, int *info,
+                                        unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err,
+                                        hipStream_t s);
 hipError_t launch_bilu0_factor_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o,
-                                        const int *order, int n, float *Mg, int *info, unsigned *flags,
-                                        unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s);
+                                        const int4 *rows, const int2 *nbr, int n, float *Mg, int *info,
+                                        unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err,
+                                        hipStream_t s);
 hipError_t launch_bilu0_syncfree(int bsz, const int4 *lrows, const int2 *lnbr, const int4 *urows, const int2 *unbr,
                                  int n, const double *Mg, const double *x, double *t, double *y, unsigned *sync,
                                  int nwg, int spin_limit, int *err, hipStream_t s);
@@ -144,12 +146,11 @@ struct SolverState {
     int order_method = -1;              // ordering behind o2u/u2o: 0 natural, 1 approximate MDF, 3 caller's
     std::vector<int> rowpts, colind;    // host copy of the trace graph
     std::vector<int> o2u, u2o;          // host copies
-    int *d_o2u = nullptr, *d_u2o = nullptr;
+    int *d_u2o = nullptr;
     std::vector<int> lptr, uptr;        // level pointers of the L (forward) and U (backward) sweeps
     std::vector<int> lrows, urows;      // rows of each level, concatenated
     std::vector<int> llev, ulev;        // level of each row
     bool sched_valid = false;           // the device copies below are the current ordering's
-    int *d_lrows = nullptr;             // lrows: the factorisation's order
     // the sweeps' rows in level order with their neighbours (RowSched, solver.hip)
     int4 *d_lsched = nullptr, *d_usched = nullptr;
     int2 *d_lnbr = nullptr, *d_unbr = nullptr;

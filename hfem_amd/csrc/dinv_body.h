@@ -102,6 +102,182 @@ template <> struct GJ<float> {
     }
 };
 
+// Key of a pivot candidate: grows with |v|; 1 for NaN.
+__device__ __forceinline__ unsigned pivot_key(double v)
+{
+    const unsigned h = (unsigned)__double2hiint(v) & 0x7fffffffu;
+    return h > 0x7ff00000u ? 1u : h + 2u;
+}
+__device__ __forceinline__ unsigned pivot_key(float v)
+{
+    const unsigned h = __float_as_uint(v) & 0x7fffffffu;
+    return h > 0x7f800000u ? 1u : h + 2u;
+}
+
+// The maximum over the wave in six DPP steps, 0 where no lane comes in; lane 63 ends
+// with it.
+template <int STEP>
+__device__ __forceinline__ unsigned key_max_step(unsigned v)
+{
+    constexpr int ctrl = STEP == 0 ? 0x111 : STEP == 1 ? 0x112 : STEP == 2 ? 0x114 : STEP == 3 ? 0x118 : STEP == 4 ? 0x142 : 0x143;
+    constexpr int rows = STEP == 4 ? 0xa : STEP == 5 ? 0xc : 0xf;   // row_shr 1, 2, 4, 8, row_bcast 15, 31
+    return max(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, rows, 0xf, false));
+}
+__device__ __forceinline__ unsigned wave_max_key(unsigned v)
+{
+    v = key_max_step<0>(v);
+    v = key_max_step<1>(v);
+    v = key_max_step<2>(v);
+    v = key_max_step<3>(v);
+    v = key_max_step<4>(v);
+    v = key_max_step<5>(v);
+    return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The pivot steps of a panel of 16 columns on one wave, the lane holding rows lane + 64 q.
+// Rows are never moved: step k takes as pivot the open row p of largest |a(i, k)| (compared
+// by the high words: up to 2^-20 relative; the lowest row on ties; a NaN only if nothing
+// else is left) and subtracts g_i = a(i, k) / a(p, k) times row p from every other row.
+// Pivot rows are not scaled here (g has the same meaning for them): the caller multiplies
+// row i by scale[i] at the end, so a column costs one FMA per row.
+//
+// The steps are a dependent chain on one wave, whose time is the latency of its parts:
+// the update of the next column, the search in it (six DPP maxima, the ballot, the
+// pivot's broadcast and reciprocal), the multipliers.  The other columns are updated
+// meanwhile, with row p's entries out of LDS (written by its lane, read by all; two
+// readlanes per column and step measured the same).  The columns rotate through the
+// registers: column k is always in x[0], updates write one register down, the multipliers
+// enter at x[15], so that the loop stays rolled.
+template <typename T, int RPL>
+struct PanelState {
+    unsigned open[RPL];   // ~0: the row can still be a pivot
+    T scale[RPL];         // 1 / pivot of the row
+    int lab[RPL];         // step at which the row was the pivot, -1 before
+    int sing;             // 1 + the first step with a zero pivot, 0: none
+    __device__ __forceinline__ void init(int n)
+    {
+        sing = 0;
+#pragma unroll
+        for (int q = 0; q < RPL; q++) {
+            open[q] = (int)(threadIdx.x & 63) + 64 * q < n ? ~0u : 0u;
+            scale[q] = (T)0;
+            lab[q] = -1;
+        }
+    }
+};
+
+// w <= 16 steps, the first of them step k0 of the matrix.  buf: 2 x 16 T of LDS, 16-byte
+// aligned.  Returns to lane k the pivot row of step k; column k of the panel is left in
+// x[16 - w + k].
+template <typename T, int RPL>
+__device__ __forceinline__ int panel_steps(T (&x)[16][RPL], int w, int k0, PanelState<T, RPL> &s, T *buf)
+{
+    typedef GJ<T> G;
+    const int lane = threadIdx.x & 63;
+    int pcv = 0;
+    unsigned key[RPL], m = 0;
+    int p = 0;
+    T pv = (T)0, pinv = (T)0, g[RPL];
+#pragma unroll
+    for (int q = 0; q < RPL; q++) {
+        key[q] = 0;
+        g[q] = (T)0;
+    }
+    auto bcast = [&](const T (&col)[RPL], int row) {
+        if constexpr (RPL == 1) return G::bcast(col[0], row);
+        else return G::bcast(row < 64 ? col[0] : col[1], row & 63);
+    };
+    constexpr int NS = 8;
+    auto search = [&](int stage, const T (&col)[RPL]) {
+        switch (stage) {
+        case 0:
+#pragma unroll
+            for (int q = 0; q < RPL; q++) key[q] = pivot_key(col[q]) & s.open[q];
+            m = key[0];
+#pragma unroll
+            for (int q = 1; q < RPL; q++) m = max(m, key[q]);
+            m = key_max_step<0>(m);
+            break;
+        case 1: m = key_max_step<1>(m); m = key_max_step<2>(m); break;
+        case 2: m = key_max_step<3>(m); m = key_max_step<4>(m); break;
+        case 3: m = key_max_step<5>(m); break;
+        case 4: {
+            const unsigned mm = (unsigned)__builtin_amdgcn_readlane((int)m, 63);
+#pragma unroll
+            for (int q = RPL - 1; q >= 0; q--) {
+                const unsigned long long b = __ballot(key[q] == mm);
+                p = b ? 64 * q + __ffsll((long long)b) - 1 : p;
+            }
+            break;
+        }
+        case 5: pv = bcast(col, p); break;
+        case 6: pinv = G::recip(pv); break;
+        case 7:
+            pinv = pv == (T)0 ? (T)0 : pinv;
+#pragma unroll
+            for (int q = 0; q < RPL; q++) g[q] = lane + 64 * q == p ? (T)0 : col[q] * pinv;
+            break;
+        }
+    };
+#pragma unroll
+    for (int st = 0; st < NS; st++) search(st, x[0]);
+#pragma unroll 1
+    for (int k = 0; k < w; k++) {
+        bool mine[RPL];
+        T gk[RPL];
+        // row p, columns 2-15, to LDS (its lane) and back (all)
+        T *row = buf + (k & 1) * 16;
+#pragma unroll
+        for (int q = 0; q < RPL; q++)
+            if (lane + 64 * q == p)
+#pragma unroll
+                for (int j = 2; j < 16; j++) row[j] = x[j][q];
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        T pr[16];
+#pragma unroll
+        for (int j = 2; j < 16; j++) pr[j] = row[j];
+        const T pr1 = bcast(x[1], p);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 0; q < RPL; q++) {
+            mine[q] = lane + 64 * q == p;
+            gk[q] = g[q];
+            x[0][q] = x[1][q] - gk[q] * pr1;
+            s.open[q] = mine[q] ? 0u : s.open[q];
+        }
+        const int pk = p;
+        const T pvk = pv, pinvk = pinv;
+        // (after the last step: of a column that is none, unused)
+#pragma unroll
+        for (int st = 0; st < NS; st++) {
+            search(st, x[0]);
+            __builtin_amdgcn_sched_barrier(0);
+            if (st == 1) {
+#pragma unroll
+                for (int q = 0; q < RPL; q++) {
+                    s.scale[q] = mine[q] ? pinvk : s.scale[q];
+                    s.lab[q] = mine[q] ? k0 + k : s.lab[q];
+                }
+                s.sing = pvk == (T)0 && !s.sing ? k0 + k + 1 : s.sing;
+                pcv = lane == k ? pk : pcv;
+            }
+            if (st >= 3) {
+                // columns 2-15 over the last five stages
+#pragma unroll
+                for (int j = 2 + 3 * (st - 3); j < 5 + 3 * (st - 3) && j < 16; j++)
+#pragma unroll
+                    for (int q = 0; q < RPL; q++) x[j - 1][q] = x[j][q] - gk[q] * pr[j];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = 0; q < RPL; q++) x[15][q] = mine[q] ? (T)1 : -gk[q];
+    }
+    return pcv;
+}
+
 // ---------------------------------------------------------------------------
 // inv(D) by blocked Gauss-Jordan on the MFMA, in arithmetic T (FP64, or FP32
 // for the mixed condensation: D is rounded to FP32 on the way in), written in

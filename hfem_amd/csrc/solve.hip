@@ -138,20 +138,16 @@ static int ensure_schedule(hfem_ctx *c)
     std::vector<int2> lnbr, unbr;
     schedule(s.lrows, s.llev, true, lsched, lnbr);
     schedule(s.urows, s.ulev, false, usched, unbr);
-    if (!s.d_lrows) HIPCHK(hfem_dalloc(&s.d_lrows, (size_t)n));
     if (!s.d_lsched) HIPCHK(hfem_dalloc(&s.d_lsched, (size_t)n));
     if (!s.d_usched) HIPCHK(hfem_dalloc(&s.d_usched, (size_t)n));
     // (each holds at most every off-diagonal block)
     if (!s.d_lnbr) HIPCHK(hfem_dalloc(&s.d_lnbr, ci.size()));
     if (!s.d_unbr) HIPCHK(hfem_dalloc(&s.d_unbr, ci.size()));
-    if (!s.d_o2u) HIPCHK(hfem_dalloc(&s.d_o2u, (size_t)n));
     if (!s.d_u2o) HIPCHK(hfem_dalloc(&s.d_u2o, (size_t)n));
-    HIPCHK(hipMemcpy(s.d_lrows, s.lrows.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s.d_lsched, lsched.data(), sizeof(int4) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s.d_usched, usched.data(), sizeof(int4) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s.d_lnbr, lnbr.data(), sizeof(int2) * lnbr.size(), hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s.d_unbr, unbr.data(), sizeof(int2) * unbr.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(s.d_o2u, s.o2u.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     HIPCHK(hipMemcpy(s.d_u2o, s.u2o.data(), sizeof(int) * n, hipMemcpyHostToDevice));
     s.sched_valid = true;
     return 0;
@@ -294,7 +290,7 @@ extern "C" int hfem_precond_factor(hfem_ctx *c, int kind)
         s.prec = -1;
         return 0;
     }
-    if ((size_t)(kind == 0 ? bilu0_factor_lds(bsz) + 16 : block_inverse_lds(bsz)) > (size_t)c->maxlds)
+    if ((size_t)(kind == 0 ? bilu0_factor_lds(bsz) : block_inverse_lds(bsz)) > (size_t)c->maxlds)
         return hfem_fail(-1, "hfem_precond_factor: block size %d needs more LDS than the device offers", bsz);
     const bool fp32 = s.prec_fp32 != 0;
     s.prec = -2;   // until this factorisation has succeeded
@@ -318,24 +314,24 @@ extern "C" int hfem_precond_factor(hfem_ctx *c, int kind)
         if (!fp32) {
             HIPCHK(hipMemcpyAsync(s.Mg, c->Hg, sizeof(double) * c->nblocks * b2, hipMemcpyDeviceToDevice, c->stream));
             if (s.sweep_mode == 1)
-                HIPCHK(launch_bilu0_factor_syncfree(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lrows, n, s.Mg, s.d_info,
+                HIPCHK(launch_bilu0_factor_syncfree(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lsched, s.d_lnbr, n, s.Mg, s.d_info,
                                                     s.sf_flags, sync, s.sweep_wgs, s.spin_limit, s.sf_err, c->stream));
             else
                 for (size_t l = 0; l + 1 < s.lptr.size(); l++)
-                    HIPCHK(launch_bilu0_factor_level(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lrows + s.lptr[l],
-                                                     s.lptr[l + 1] - s.lptr[l], s.Mg, s.d_info, c->stream));
+                    HIPCHK(launch_bilu0_factor_level(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lsched, s.d_lnbr,
+                                                     s.lptr[l], s.lptr[l + 1], s.Mg, s.d_info, c->stream));
         } else {
             // single precision (precPrecision 0): Hg rounded to FP32 and factored on
             // the FP32 MFMA
             HIPCHK(launch_to_float((long)c->nblocks * b2, c->Hg, s.Mg32, c->stream));
             if (s.sweep_mode == 1)
-                HIPCHK(launch_bilu0_factor_syncfree(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lrows, n, s.Mg32,
+                HIPCHK(launch_bilu0_factor_syncfree(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lsched, s.d_lnbr, n, s.Mg32,
                                                     s.d_info, s.sf_flags, sync, s.sweep_wgs, s.spin_limit, s.sf_err,
                                                     c->stream));
             else
                 for (size_t l = 0; l + 1 < s.lptr.size(); l++)
-                    HIPCHK(launch_bilu0_factor_level(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lrows + s.lptr[l],
-                                                     s.lptr[l + 1] - s.lptr[l], s.Mg32, s.d_info, c->stream));
+                    HIPCHK(launch_bilu0_factor_level(bsz, c->rowstart, c->cols, s.d_u2o, s.d_lsched, s.d_lnbr,
+                                                     s.lptr[l], s.lptr[l + 1], s.Mg32, s.d_info, c->stream));
         }
     }
     if (kind != 2) {

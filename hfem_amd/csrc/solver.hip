@@ -5,6 +5,7 @@
 //
 // BSR blocks are bsz x bsz column-major, rows = faces, the diagonal block first in
 // each row (the reference's Hg layout, assembly/globalassembly.cpp:42-86).
+#include "dinv_body.h"
 #include "hfem_device.h"
 
 #include <algorithm>
@@ -13,174 +14,249 @@
 namespace hfem {
 
 constexpr int SV_THREADS = 256;
-constexpr int ELIM_BATCH = 8;   // block-inverse entries a thread updates per batch
 
-// A lane's value from lane l - s (DPP control CTRL, rows in ROWS); lanes without
-// a source keep idv.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_take(double idv, double v)
+constexpr int FACTOR_MAXROW = 64;     // longest BSR row the factorisation takes
+
+// A lane index the compiler cannot see through: address arithmetic formed from it stays
+// where it is used (hoisted out of the row loops it fills the registers).
+__device__ __forceinline__ int opaque(int v)
 {
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(idv), __double2hiint(v), CTRL, ROWS, 0xf, false);
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(idv), __double2loint(v), CTRL, ROWS, 0xf, false);
-    return __hiloint2double(hi, lo);
-}
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float dpp_take(float idv, float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(idv), __float_as_int(v), CTRL, ROWS, 0xf, false));
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
-// One step of the pivot choice's scan: (b, i) becomes the better of itself and
-// the pair DPP brings in -- the larger value, the smaller row on ties -- with
-// (-1, k) where no pair comes in (the search's starting pair: no row of column k
-// has a magnitude below 0, and a NaN never replaces it).
-template <int CTRL, int ROWS, typename T>
-__device__ __forceinline__ void argmax_step(T &b, int &i, int k)
-{
-    const T yb = dpp_take<CTRL, ROWS>((T)-1, b);
-    const int yi = __builtin_amdgcn_update_dpp(k, i, CTRL, ROWS, 0xf, false);
-    const bool t = yb > b || (yb == b && yi < i);
-    b = t ? yb : b;
-    i = t ? yi : i;
-}
-
-// In-place Gauss-Jordan inverse of an n x n column-major block in LDS with
-// partial pivoting: rows are interchanged as pivots are chosen and the columns of
-// the result unscrambled in reverse order at the end.  All threads of the
-// workgroup call it; piv (n ints), rowk/colk (n values each) and red (1 value)
-// are LDS; T is the arithmetic (double, or float for FP32 preconditioner factors).
-// LATENCY picks the elimination for an inverse on a dependency chain (batched
-// reads, no branches per entry: the BILU0 factorisations) over the one for many
-// independent blocks per CU (one entry at a time, fewer registers: the block-Jacobi
-// and MDF inverses); both compute the same values.
-// Returns 0, or 1 + the step of the first zero pivot (workgroup-uniform).
-template <typename T, bool LATENCY = true>
-__device__ int lds_inverse(T *A, int n, int *piv, T *rowk, T *colk, T *red)
-{
-    const int tid = threadIdx.x, nth = blockDim.x;
-    // idx / n as a multiply-high by ceil(2^32 / n): exact for every idx < n * n
-    // with n <= 128 (checked exhaustively); n = 1 gives 0, and idx is 0 there
-    const unsigned ndiv = (unsigned)((0x100000000ull + (unsigned)n - 1) / (unsigned)n);
-    for (int k = 0; k < n; k++) {
-        if (tid < 64) {
-            T best = (T)-1;
-            int bi = k;
-            for (int i = k + tid; i < n; i += 64) {
-                const T v = fabs(A[i + n * k]);
-                if (v > best) { best = v; bi = i; }
-            }
-            // inclusive scan over the wave by DPP: shifts by 1, 2, 4, 8 within each
-            // row of 16 lanes, then row 0's total into row 1 and row 2's into row 3,
-            // then lanes 0-31's total into rows 2 and 3: lane 63 ends with the choice
-            argmax_step<0x111, 0xf>(best, bi, k);   // row_shr:1
-            argmax_step<0x112, 0xf>(best, bi, k);   // row_shr:2
-            argmax_step<0x114, 0xf>(best, bi, k);   // row_shr:4
-            argmax_step<0x118, 0xf>(best, bi, k);   // row_shr:8
-            argmax_step<0x142, 0xa>(best, bi, k);   // row_bcast:15
-            argmax_step<0x143, 0xc>(best, bi, k);   // row_bcast:31
-            if (tid == 63) { piv[k] = bi; red[0] = best; }
-        }
-        __syncthreads();
-        if (red[0] == (T)0) return k + 1;
-        const int p = piv[k];
-        for (int j = tid; j < n; j += nth) {
-            T a = A[k + n * j], b = A[p + n * j];
-            rowk[j] = b;                         // pivot row after the interchange
-            if (p != k) { A[k + n * j] = b; A[p + n * j] = a; }
-        }
-        __syncthreads();
-        for (int i = tid; i < n; i += nth) colk[i] = A[i + n * k];
-        __syncthreads();
-        const T pinv = (T)1 / rowk[k];
-        if (!LATENCY) {
-            // many blocks per CU (throughput): one entry at a time, fewer registers
-            for (int idx = tid; idx < n * n; idx += nth) {
-                const int j = idx / n, i = idx - j * n;
-                T v;
-                if (i == k) v = (j == k) ? pinv : rowk[j] * pinv;
-                else if (j == k) v = -colk[i] * pinv;
-                else v = A[idx] - colk[i] * (rowk[j] * pinv);
-                A[idx] = v;
-            }
-        }
-        // a thread's entries idx = tid + u * nth in batches of ELIM_BATCH: every read
-        // of a batch is issued before its first write, so the LDS latency is paid
-        // once per batch rather than once per entry
-        for (int base = tid; LATENCY && base < n * n; base += ELIM_BATCH * nth) {
-            T a[ELIM_BATCH], c[ELIM_BATCH], rw[ELIM_BATCH];
-            bool rk[ELIM_BATCH], ck[ELIM_BATCH];
-#pragma unroll
-            for (int u = 0; u < ELIM_BATCH; u++) {
-                // (an entry past the block reads entry 0's operands and is not stored)
-                const int idx = base + u * nth < n * n ? base + u * nth : 0;
-                const int j = (int)__umulhi((unsigned)idx, ndiv), i = idx - j * n;
-                rk[u] = i == k;
-                ck[u] = j == k;
-                a[u] = A[idx];
-                c[u] = colk[i];
-                rw[u] = rowk[j];
-            }
-            // the three cases computed alike and selected (no branches per entry)
-#pragma unroll
-            for (int u = 0; u < ELIM_BATCH; u++) {
-                const int idx = base + u * nth;
-                const T rp = rw[u] * pinv;
-                const T other = a[u] - c[u] * rp;
-                const T colv = -c[u] * pinv;
-                const T v = rk[u] ? (ck[u] ? pinv : rp) : (ck[u] ? colv : other);
-                if (idx < n * n) A[idx] = v;
-            }
-        }
-        __syncthreads();
+// MFMA 16x16x4 operands: lane l supplies A(l%16, l/16) and B(l/16, l%16); result lane l,
+// element v holds C(l/16 + 4v, l%16) (FP64) or C(4(l/16) + v, l%16) (FP32).
+template <typename T> struct BlkMfma;
+template <> struct BlkMfma<double> {
+    typedef double v4 __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ v4 run(double a, double b, v4 c)
+    {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
     }
-    for (int k = n - 1; k >= 0; k--) {
-        const int p = piv[k];
-        if (p != k)
-            for (int i = tid; i < n; i += nth) {
-                T t = A[i + n * k];
-                A[i + n * k] = A[i + n * p];
-                A[i + n * p] = t;
-            }
-        __syncthreads();
+    static __device__ __forceinline__ int row(int lk, int v) { return lk + 4 * v; }
+};
+template <> struct BlkMfma<float> {
+    typedef float v4 __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ v4 run(float a, float b, v4 c)
+    {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
     }
-    return 0;
-}
-
-template <typename T> struct LdsInv {
-    T *rowk, *colk, *red;
-    int *piv;
+    static __device__ __forceinline__ int row(int lk, int v) { return 4 * lk + v; }
 };
 
+// ---- inverse of one block ----
+//
+// Blocked Gauss-Jordan with partial pivoting of an n x n block in LDS (column-major,
+// stride n), in place up to the permutation and the row scales, by a workgroup of four
+// waves.  Per panel of 16 columns wave 0 runs the pivot steps in registers (panel_steps,
+// dinv_body.h); the panel then holds Gp = T(:, P), T the product of its elementary steps
+// and P its pivot rows, and every other column a becomes T a = Abar + Gp a(P), Abar = a
+// with the rows P zeroed: rank-16 updates of 16 x 16 tiles on the MFMA.
+// In the BILU0 factorisation the inverse stands on the chain of dependent rows, so wave 0
+// updates the next panel's columns itself and goes on while the other waves update the
+// rest: one barrier per panel.  What the others do during the pivot steps is the
+// caller's (idle(), by waves 1-3 once per panel).
+// 45 x 45 FP64, alone on its CU: 23 us, of which the chain of the 45 pivot steps 15 us
+// (0.33 us each) and wave 0's updates 2.4 us; with the block in LDS and a barrier around
+// every pass (the earlier form) 95 us.
+//
+// LDS besides the block: the rows' scales, a pivot row's entries on their way (twice),
+// per panel's parity the set of its pivot rows and the pivot rows of its steps, per row
+// its step, per step its row, and a flag.
 template <typename T>
-__device__ LdsInv<T> lds_inv_area(T *p, int n)
+struct InvShared {
+    static constexpr int head(int rows) { return (int)((rows * sizeof(T) + 15) / 16 * 16); }
+    static constexpr int bytes(int rows) { return head(rows) + 2 * 16 * (int)sizeof(T) + 4 * 8 + (2 * 16 + 2 * rows + 1) * 4; }
+    T *scale, *buf;
+    unsigned long long *set;
+    int *prow, *lab, *pof, *sing;
+    // mem: 16-byte aligned
+    __device__ InvShared(void *mem, int rows)
+    {
+        scale = (T *)mem;
+        buf = (T *)((char *)mem + head(rows));
+        set = (unsigned long long *)(buf + 2 * 16);
+        prow = (int *)(set + 4);
+        lab = prow + 2 * 16;
+        pof = lab + rows;
+        sing = pof + rows;
+    }
+};
+
+// NT: 16-row tiles (at least ceil(n / 16)).
+// All threads call it with the block complete (a barrier before); out(i, c, v) receives
+// every entry of the inverse once, rows along the lanes.  Returns 0, or 1 + the step of
+// the first zero pivot (workgroup-uniform; the result is then finite but no inverse).
+template <typename T, int NT, class IDLE, class OUT>
+__device__ __forceinline__ int wg_inverse(int n, T *A, const InvShared<T> &sh, IDLE idle, OUT out)
 {
-    LdsInv<T> w;
-    w.rowk = p;
-    w.colk = p + n;
-    w.red = p + 2 * n;
-    w.piv = (int *)(p + 2 * n + 2);
-    return w;
+    typedef BlkMfma<T> M;
+    typedef typename M::v4 v4;
+    constexpr int RPL = NT <= 4 ? 1 : 2;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt = (n + 15) / 16;
+    PanelState<T, RPL> ps;
+    if (wv == 0) ps.init(n);
+    // panel pb's update of tile column ct
+    auto update = [&](int pb, int ct) {
+        const int lr = opaque(lane & 15), lk = opaque(lane >> 4);
+        const int kw = min(16, n - 16 * pb), col = min(16 * ct + lr, n - 1);
+        const int *prow = sh.prow + (pb & 1) * 16;
+        T *C = A + n * col;
+        T b[4];
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            const int k = 4 * ks + lk;
+            b[ks] = C[prow[min(k, kw - 1)]];
+            b[ks] = k < kw ? b[ks] : (T)0;
+        }
+        // the lane's rows 16 r + row(lk, v) among the pivot rows: bits 16 r + row(0, v)
+        // of the set moved down by row(lk, 0)
+        const unsigned long long set0 = sh.set[2 * (pb & 1)] >> M::row(lk, 0);
+        const unsigned long long set1 = NT > 4 ? sh.set[2 * (pb & 1) + 1] >> M::row(lk, 0) : 0;
+        v4 acc[NT];
+#pragma unroll
+        for (int r = 0; r < NT; r++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const T c = C[min(16 * r + M::row(lk, v), n - 1)];
+                const unsigned long long set = r < 4 ? set0 : set1;
+                acc[r][v] = (set >> (16 * (r & 3) + M::row(0, v))) & 1 ? (T)0 : c;
+            }
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+            const int k = min(4 * ks + lk, kw - 1);
+            T a[NT];
+#pragma unroll
+            for (int r = 0; r < NT; r++) a[r] = A[min(16 * r + lr, n - 1) + n * (16 * pb + k)];
+#pragma unroll
+            for (int r = 0; r < NT; r++) acc[r] = M::run(a[r], b[ks], acc[r]);
+        }
+        // (this wave alone touches the tile column between two barriers)
+#pragma unroll
+        for (int r = 0; r < NT; r++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = 16 * r + M::row(lk, v);
+                if (i < n && 16 * ct + lr < n) C[i] = acc[r][v];
+            }
+    };
+    for (int pb = 0;; pb++) {
+        // the previous panel's update: its tile columns but the next panel's, which is wave
+        // 0's, over waves 1-3 (after the last panel over all four)
+        for (int ct = 0, d = 1; pb > 0 && ct < nt; ct++) {
+            if (ct == pb - 1) continue;
+            const int w = ct == pb ? 0 : d;
+            if (ct != pb) d = d == 3 ? pb < nt : d + 1;
+            if (wv == w) update(pb - 1, ct);
+        }
+        if (pb == nt) break;
+        if (wv == 0) {
+            const int kw = min(16, n - 16 * pb);
+            T x[16][RPL];
+#pragma unroll
+            for (int j = 0; j < 16; j++)
+#pragma unroll
+                for (int q = 0; q < RPL; q++) x[j][q] = A[min(lane + 64 * q, n - 1) + n * min(16 * pb + j, n - 1)];
+            const int pcv = panel_steps<T, RPL>(x, kw, 16 * pb, ps, sh.buf);
+            // column k of the panel is in x[16 - kw + k] after kw rotations
+            T *P = A + n * (16 * pb + kw - 16);
+#pragma unroll
+            for (int q = 0; q < RPL; q++)
+                if (lane + 64 * q < n) {
+#pragma unroll
+                    for (int j = 0; j < 16; j++)
+                        if (j >= 16 - kw) P[lane + 64 * q + n * j] = x[j][q];
+                    sh.lab[lane + 64 * q] = ps.lab[q];
+                    sh.scale[lane + 64 * q] = ps.scale[q];
+                }
+#pragma unroll
+            for (int q = 0; q < RPL; q++) {
+                const unsigned long long set = __ballot(ps.lab[q] >= 16 * pb);
+                if (lane == 0) sh.set[2 * (pb & 1) + q] = set;
+            }
+            if (lane < kw) {
+                sh.prow[(pb & 1) * 16 + lane] = pcv;
+                sh.pof[16 * pb + lane] = pcv;
+            }
+            if (lane == 0) *sh.sing = ps.sing;
+        } else {
+            idle();
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    int lab[RPL];
+    T sc[RPL];
+#pragma unroll
+    for (int q = 0; q < RPL; q++) {
+        lab[q] = sh.lab[min(lane + 64 * q, n - 1)];
+        sc[q] = sh.scale[min(lane + 64 * q, n - 1)];
+    }
+    int pof[RPL];
+#pragma unroll
+    for (int q = 0; q < RPL; q++) pof[q] = sh.pof[min(lane + 64 * q, n - 1)];
+    // the wave's columns c = wv, wv + 4, ..., four at a time
+    for (int c0 = wv; c0 < n; c0 += 16) {
+        T v[4][RPL];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int q = 0; q < RPL; q++) v[u][q] = A[min(lane + 64 * q, n - 1) + n * min(c0 + 4 * u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int c = c0 + 4 * u, cc = min(c, n - 1);
+            int pc = __builtin_amdgcn_readlane(pof[0], cc & 63);
+            if (RPL > 1 && cc >= 64) pc = __builtin_amdgcn_readlane(pof[RPL - 1], cc & 63);
+#pragma unroll
+            for (int q = 0; q < RPL; q++)
+                if (c < n && lane + 64 * q < n) out(lab[q], pc, v[u][q] * sc[q]);
+        }
+    }
+    return __builtin_amdgcn_readfirstlane(*sh.sing);
 }
 
-size_t lds_inv_bytes(int n) { return sizeof(double) * (2 * n + 2) + sizeof(int) * (n + 2); }
+// The block kernels' shapes by block size: CPW = columns per wave of four (and, for the
+// MFMA products, k-steps of 4), RCH rows per lane.  A shape's unused columns cost their
+// share of the work, so the sizes in use have one that fits: 8-16 (triangles p=1-3, tets
+// p=1), 20 and 24 (triangles p=4, 5, hexes p=1), 30 (tets p=2), 45 (hexes p=2), 50 (tets
+// p=3), 75 (tets p=4).  launch(RCH, CPW) with integral constants.
+template <class F>
+static hipError_t block_shape(int bsz, F launch)
+{
+#define SHAPE(R, C) launch(std::integral_constant<int, R>(), std::integral_constant<int, C>())
+    if (bsz < 1 || bsz > 128) return hipErrorInvalidValue;
+    if (bsz <= 16) SHAPE(1, 4);
+    else if (bsz <= 24) SHAPE(1, 6);
+    else if (bsz <= 32) SHAPE(1, 8);
+    else if (bsz <= 48) SHAPE(1, 12);
+    else if (bsz <= 52) SHAPE(1, 13);
+    else if (bsz <= 64) SHAPE(1, 16);
+    else if (bsz <= 80) SHAPE(2, 20);
+    else SHAPE(2, 32);
+#undef SHAPE
+    return hipGetLastError();
+}
 
 // Inverses of the diagonal blocks of Hg (block-Jacobi, mkBlockJacobi.m:9-11, and
-// the MDF weights).  One workgroup per row.
-__global__ void __launch_bounds__(SV_THREADS)
+// the MDF weights).  One workgroup per row.  34 104 blocks of 50 x 50: 4.6 ms with the
+// earlier LDS form, 1.26 ms now (floor: 1.4 GB in and out, 0.28 ms).
+template <int NT>
+__global__ void __launch_bounds__(SV_THREADS, NT <= 4 ? 4 : 2)
 block_inverse_kernel(int nrows, int bsz, const int *__restrict__ rowpts, const double *__restrict__ Hg,
                      double *__restrict__ Dinv, int *__restrict__ info)
 {
-    extern __shared__ double lds[];
+    extern __shared__ __align__(16) double lds[];
     const int tid = threadIdx.x, nth = blockDim.x;
     const long b2 = (long)bsz * bsz;
     double *A = lds;
-    LdsInv<double> w = lds_inv_area(A + b2, bsz);
+    const InvShared<double> sh(A + (b2 + 1) / 2 * 2, bsz);
     for (int row = blockIdx.x; row < nrows; row += gridDim.x) {
         const double *src = Hg + (long)rowpts[row] * b2;
         for (long i = tid; i < b2; i += nth) A[i] = src[i];
         __syncthreads();
-        const int r = lds_inverse<double, false>(A, bsz, w.piv, w.rowk, w.colk, w.red);
-        for (long i = tid; i < b2; i += nth) Dinv[row * b2 + i] = A[i];
+        double *dst = Dinv + row * b2;
+        const int r = wg_inverse<double, NT>(bsz, A, sh, [] {}, [&](int i, int c, double v) { dst[i + bsz * c] = v; });
         if (tid == 0 && info) info[row] = r;
         __syncthreads();
     }
@@ -217,219 +293,6 @@ mdf_weight_kernel(int nrows, int bsz, const int *__restrict__ rowpts, const doub
             if (tid == 0) Cw[n] = sqrt(red[0]);
             __syncthreads();
         }
-    }
-}
-
-// BILU0 factorisation of the rows of one level (kernel/computeBILU0.m), in the
-// row-oriented form: row ri takes, for each neighbour rk numbered before it in
-// increasing order, L_ik = A_ik inv(U_kk), then A_ii -= L_ik A_ki and A_il -=
-// L_ik A_kl for the later common neighbours rl; finally A_ii is inverted.  Each
-// block of row ri receives the same updates in the same order as in the
-// reference's right-looking loop; rows of one level do not depend on each other.
-// The column lists of row ri and of the current neighbour row sit in LDS, so the
-// neighbour order and the target search cost no memory round trips; blocks are
-// staged into LDS with eight loads in flight per thread and multiplied on the
-// FP64 MFMA.  The blocks of row ri that are read again (the targets and the
-// diagonal) are always read and written with the fixed entry -> thread map of
-// wg_load_block / wg_subtract_block, so a thread only ever re-reads global
-// entries it wrote itself; L_ik, stored from the MFMA result layout, is not read
-// again by the row.
-constexpr int FACTOR_MAXROW = 64;     // longest BSR row the factorisation takes
-
-typedef double f64x4 __attribute__((ext_vector_type(4)));
-
-// The n x n product C = A B of two column-major LDS blocks on the MFMA (FP64, or
-// FP32 for FP32 preconditioner factors): the 16 x 16 tiles of C are spread over
-// the waves, rows and columns past n are masked to zero; out(i, j, c) receives
-// each entry of C (i, j < n).  MFMA 16x16x4 operands: lane l supplies A(l%16,
-// l/16) and B(l/16, l%16); result lane l, element v holds C(l/16 + 4v, l%16)
-// (FP64) or C(4(l/16) + v, l%16) (FP32).
-template <typename T> struct BlkMfma;
-template <> struct BlkMfma<double> {
-    typedef double v4 __attribute__((ext_vector_type(4)));
-    static __device__ __forceinline__ v4 run(double a, double b, v4 c)
-    {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int lk, int v) { return lk + 4 * v; }
-};
-template <> struct BlkMfma<float> {
-    typedef float v4 __attribute__((ext_vector_type(4)));
-    static __device__ __forceinline__ v4 run(float a, float b, v4 c)
-    {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-    static __device__ __forceinline__ int row(int lk, int v) { return 4 * lk + v; }
-};
-
-template <typename T, typename OUT>
-__device__ __forceinline__ void lds_block_product(const T *A, const T *B, int n, OUT out)
-{
-    typedef BlkMfma<T> M;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nw = blockDim.x >> 6;
-    const int lr = lane & 15, lk = lane >> 4, nt = (n + 15) / 16, ntt = nt * nt;
-    // four of the wave's tiles at a time (t = tb + nw u), their MFMA chains
-    // interleaved; each tile's k order is that of one tile alone
-    constexpr int U = 4;
-    for (int tb = wave; tb < ntt; tb += U * nw) {
-        int ia[U], jb[U], i0[U], j0[U];
-        bool va[U], vb[U], tv[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) {
-            const int t0 = tb + nw * u;
-            tv[u] = t0 < ntt;
-            const int t = tv[u] ? t0 : tb;
-            i0[u] = (t % nt) * 16;
-            j0[u] = (t / nt) * 16;
-            ia[u] = min(i0[u] + lr, n - 1);
-            jb[u] = min(j0[u] + lr, n - 1);
-            va[u] = i0[u] + lr < n;
-            vb[u] = j0[u] + lr < n;
-        }
-        typename M::v4 acc[U];
-#pragma unroll
-        for (int u = 0; u < U; u++) acc[u] = (typename M::v4){(T)0, (T)0, (T)0, (T)0};
-        for (int k0 = 0; k0 < n; k0 += 4) {
-            const int k = k0 + lk, kc = min(k, n - 1);
-            T a[U], b[U];
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                a[u] = (va[u] && k < n) ? A[ia[u] + n * kc] : (T)0;
-                b[u] = (vb[u] && k < n) ? B[kc + n * jb[u]] : (T)0;
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) acc[u] = M::run(a[u], b[u], acc[u]);
-        }
-#pragma unroll
-        for (int u = 0; u < U; u++)
-#pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int i = i0[u] + M::row(lk, v), j = j0[u] + lr;
-                if (tv[u] && i < n && j < n) out(i, j, acc[u][v]);
-            }
-    }
-}
-
-// dst[i] = src[i] for i < n (n >= 1) by the workgroup, eight loads in flight per
-// thread (addresses clamped into the block).  Entry i is always handled by thread
-// i % blockDim.x.
-template <typename T>
-__device__ __forceinline__ void wg_load_block(T *dst, const T *__restrict__ src, long n)
-{
-    const int tid = threadIdx.x, nth = blockDim.x;
-    for (long b = tid; b < n; b += 8L * nth) {
-        T v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = src[min(b + (long)j * nth, n - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (b + (long)j * nth < n) dst[b + (long)j * nth] = v[j];
-    }
-}
-
-// dst[i] -= d[i] for i < n, global dst, LDS d; same entry -> thread map as
-// wg_load_block.
-template <typename T>
-__device__ __forceinline__ void wg_subtract_block(T *dst, const T *d, long n)
-{
-    const int tid = threadIdx.x, nth = blockDim.x;
-    for (long b = tid; b < n; b += 8L * nth) {
-        T v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = dst[min(b + (long)j * nth, n - 1)];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (b + (long)j * nth < n) dst[b + (long)j * nth] = v[j] - d[b + (long)j * nth];
-    }
-}
-
-// T: the factors' type (double, or float: the reference's single-precision
-// preconditioner, precPrecision 0, preprocessing/initializestructs.cpp:476-486,
-// factored here on the FP32 MFMA).
-template <typename T>
-__global__ void __launch_bounds__(SV_THREADS)
-bilu0_factor_kernel(int bsz, const int *__restrict__ rowpts, const int *__restrict__ colind,
-                    const int *__restrict__ u2o, const int *__restrict__ rows, int nlev, T *__restrict__ Mg,
-                    int *__restrict__ info)
-{
-    extern __shared__ double lds_raw[];
-    T *lds = (T *)lds_raw;
-    const int tid = threadIdx.x, nth = blockDim.x;
-    const long b2 = (long)bsz * bsz;
-    T *X = lds, *B = lds + b2, *L = lds + 2 * b2;
-    LdsInv<T> w = lds_inv_area(lds + 3 * b2, bsz);
-    // row ri: columns and their order numbers; the lower neighbours' positions by
-    // increasing order number; the current neighbour row's columns
-    int *rcol = w.piv + bsz + 2, *rord = rcol + FACTOR_MAXROW, *lst = rord + FACTOR_MAXROW,
-        *ncol = lst + FACTOR_MAXROW + 1;
-    for (int t = blockIdx.x; t < nlev; t += gridDim.x) {
-        const int ri = rows[t], oi = u2o[ri], d0 = rowpts[ri], len = rowpts[ri + 1] - d0;
-        if (len > FACTOR_MAXROW) {
-            // workgroup-uniform: reported through info, the row is left as it is
-            if (tid == 0) info[ri] = -len;
-            continue;
-        }
-        if (tid < len) {
-            const int c = colind[d0 + tid];
-            rcol[tid] = c;
-            rord[tid] = u2o[c];
-        }
-        __syncthreads();
-        if (tid == 0) {
-            int cnt = 0;
-            for (int q = 1; q < len; q++) {
-                if (rord[q] >= oi) continue;
-                int m = cnt++;                    // insertion by increasing order number
-                while (m > 0 && rord[lst[1 + m - 1]] > rord[q]) {
-                    lst[1 + m] = lst[1 + m - 1];
-                    m--;
-                }
-                lst[1 + m] = q;
-            }
-            lst[0] = cnt;
-        }
-        __syncthreads();
-        const int cnt = lst[0];
-        for (int qq = 0; qq < cnt; qq++) {
-            const int q = lst[1 + qq], ik = d0 + q, rk = rcol[q], ork = rord[q];
-            const int k0 = rowpts[rk], klen = rowpts[rk + 1] - k0;
-            if (tid < klen && tid < FACTOR_MAXROW) ncol[tid] = colind[k0 + tid];
-            wg_load_block(X, Mg + (long)ik * b2, b2);
-            wg_load_block(B, Mg + (long)k0 * b2, b2);     // inv(U_kk)
-            __syncthreads();
-            // L_ik = A_ik inv(U_kk), kept in LDS and stored in place of A_ik
-            T *Mik = Mg + (long)ik * b2;
-            lds_block_product(X, B, bsz, [&](int i, int j, T c) {
-                L[i + bsz * j] = c;
-                Mik[i + bsz * j] = c;
-            });
-            __syncthreads();
-            // targets in row ri: the diagonal (source: ri's position in row rk) and the
-            // later common neighbours rl (source: rl's position in row rk)
-            for (int l = 0; l < len; l++) {
-                if (l != 0 && rord[l] <= ork) continue;
-                const int rl = rcol[l];
-                int km = -1;
-                for (int m = 1; m < klen && m < FACTOR_MAXROW; m++)
-                    if (ncol[m] == rl) { km = m; break; }
-                if (km < 0) continue;
-                wg_load_block(B, Mg + (long)(k0 + km) * b2, b2);
-                __syncthreads();
-                lds_block_product(L, B, bsz, [&](int i, int j, T c) { X[i + bsz * j] = c; });
-                __syncthreads();
-                wg_subtract_block(Mg + (long)(d0 + l) * b2, X, b2);
-                __syncthreads();
-            }
-            // targets skipped above run no barrier: every wave must be done scanning
-            // ncol before the next neighbour's column list overwrites it
-            __syncthreads();
-        }
-        wg_load_block(X, Mg + (long)d0 * b2, b2);
-        __syncthreads();
-        const int r = lds_inverse(X, bsz, w.piv, w.rowk, w.colk, w.red);
-        for (long i = tid; i < b2; i += nth) Mg[(long)d0 * b2 + i] = X[i];
-        if (tid == 0) info[ri] = r;
-        __syncthreads();
     }
 }
 
@@ -688,26 +551,6 @@ sweep_reset_kernel(unsigned *sync, long n, double *t, double *y)
     }
 }
 
-// Wait until *f holds `epoch`, for the factorisation's ready flags.  The flags and
-// the blocks they guard are read and written only by agent-scope atomics (coherent
-// across the XCDs without whole-L2 write-backs or invalidations, which an acquire /
-// release pair costs here per row).  At most spin_limit polls; a wait that runs out,
-// or any wait once another has (*err set), sets *err and returns.
-__device__ __forceinline__ void wait_ready(const unsigned *f, unsigned epoch, int spin_limit, int *err)
-{
-    // (the polled values go through readfirstlane: a uniform loop)
-    int spins = 0;
-    while ((unsigned)__builtin_amdgcn_readfirstlane(
-               __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != epoch) {
-        if (++spins > spin_limit ||
-            __builtin_amdgcn_readfirstlane(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) {
-            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return;
-        }
-        __builtin_amdgcn_s_sleep(2);
-    }
-}
-
 // The factorisation's last step for the sweeps: every upper block of row r becomes
 // U~_rl = inv(U_rr) U_rl (inv(U_rr) is the row's diagonal block), in place, after
 // the whole factorisation (the other rows' eliminations read the unscaled U_rl).
@@ -750,6 +593,364 @@ bilu0_scale_upper_kernel(int bsz, int n, const int *__restrict__ rowpts, const i
     }
 }
 
+// ---- BILU0 factorisation (kernel/computeBILU0.m) ----
+//
+// In the row-oriented form: row i takes, for each neighbour k numbered before it,
+// L_ik = A_ik inv(U_kk), then A_ii -= L_ik U_ki and A_il -= L_ik U_kl for the later
+// common neighbours l; finally A_ii is inverted.  The neighbours go by level: adjacent
+// rows have different levels, in the order of their numbers, so every block receives
+// its updates in an order the right-looking loop allows.
+//
+// Bound by its chain of dependent rows, like the sweeps (at 16 464 p=3 tets 557 links;
+// its products would take 3 ms), so a row is laid out for the time from its last
+// neighbour's flag to its own:
+// * One workgroup of four waves per row.  The products run on the MFMA, 16 x 16 tiles;
+//   a wave takes whole tile columns, so its B operands (inv(U_kk), U_kl) go from memory
+//   straight into registers, all k-steps in flight, with no barrier behind the flag.
+//   The A operands are in LDS: A_ik, staged before the wait, and -L_ik.
+// * U_ki is fetched with inv(U_kk), each further target's operands during the product
+//   before it.
+// * The diagonal block stays in LDS until it is inverted there (wg_inverse); the last
+//   neighbour's other targets are updated in that inverse's idle phases.
+// * Which blocks are targets is found in registers (the column list of row k against
+//   that of row i, lane by lane), before the wait.
+// Blocks that other rows read go through agent-scope atomics (coherent across the
+// XCDs); the row's flag is stored after every wave's stores have completed.
+// FP64, before (all operands through LDS, target search by LDS scans, the inverse in
+// LDS) and now: 16 464 p=3 tets (block 50, 557 levels) 86.9 and 27.0 ms; 8^3 periodic p=2
+// hexes (block 45, 370 levels) 43.1 and 11.5 ms; 4 608 p=4 triangles (block 25, 849
+// levels) 37.2 and 11.9 ms.  Of a row's time in the hexes (28 us): its first neighbour's
+// flag to L 3.4 us, the targets 2.4 us, the inverse 22 us.
+
+// Wait until *f holds `epoch`, for the factorisation's ready flags.  At most
+// spin_limit polls; a wait that runs out, or any wait once another has (*err set), sets
+// *err and returns.
+__device__ __forceinline__ void wait_ready(const unsigned *f, unsigned epoch, int spin_limit, int *err)
+{
+    // (the polled values go through readfirstlane: a uniform loop)
+    int spins = 0;
+    while ((unsigned)__builtin_amdgcn_readfirstlane(
+               __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != epoch) {
+        if (++spins > spin_limit ||
+            ((spins & 63) == 0 && __builtin_amdgcn_readfirstlane(
+                                      __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))) {
+            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return;
+        }
+        __builtin_amdgcn_s_sleep(1);
+    }
+}
+
+// Entry o of a block: a uniform base and an unsigned byte offset, so that a block's
+// addresses are one register each.
+template <typename T>
+__device__ __forceinline__ T *entry(T *base, int o)
+{
+    return (T *)((char *)base + (unsigned)o * (unsigned)sizeof(T));
+}
+template <typename T>
+__device__ __forceinline__ const T *entry(const T *base, int o)
+{
+    return (const T *)((const char *)base + (unsigned)o * (unsigned)sizeof(T));
+}
+template <typename T>
+__device__ __forceinline__ T coh_load(const T *base, int o)
+{
+    return __hip_atomic_load(entry(base, o), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T>
+__device__ __forceinline__ void coh_store(T *base, int o, T v)
+{
+    __hip_atomic_store(entry(base, o), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The workgroup's tiles of an n x n block product on the MFMA: NT = ceil(CPW / 4) tiles
+// a side.  A wave takes tile column `wave` (NT 3, 4; NT 1: the first wave alone), one
+// tile of four (NT 2), or tile column `wave` and its share of the fifth (NT 5).
+template <typename T, int CPW>
+struct BlockTiles {
+    typedef BlkMfma<T> M;
+    typedef typename M::v4 v4;
+    static constexpr int NT = (CPW + 3) / 4, NCB = NT == 5 ? 2 : 1, TPW = NT <= 2 ? 1 : NT <= 4 ? NT : 7;
+    static_assert(NT <= 5, "block size");
+    int n, lr, lk, wv;
+    __device__ BlockTiles(int n_) : n(n_)
+    {
+        const int lane = threadIdx.x & 63;
+        lr = lane & 15;
+        lk = lane >> 4;
+        wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    }
+    __device__ bool active() const { return NT == 1 ? wv == 0 : NT == 3 ? wv < 3 : true; }
+    __device__ bool has(int s) const { return s < 6 || wv == 0; }
+    __device__ int rt(int s) const { return NT == 2 ? wv >> 1 : s < 5 ? s : s == 5 ? wv : 4; }
+    __device__ int cb(int s) const { return s < 5 ? 0 : 1; }
+    __device__ int ct(int b) const { return b ? 4 : NT == 2 ? (wv & 1) : wv; }
+    // B operands: every k-step of the wave's tile columns of a block in global memory
+    __device__ __forceinline__ void load_b(const T *B, T (&b)[NCB][CPW]) const
+    {
+#pragma unroll
+        for (int c = 0; c < NCB; c++) {
+            const int col = min(ct(c) * 16 + opaque(lr), n - 1), k = opaque(lk);
+#pragma unroll
+            for (int ks = 0; ks < CPW; ks++) b[c][ks] = coh_load(B, min(4 * ks + k, n - 1) + n * col);
+        }
+    }
+    // acc += A b with A in LDS (rows past n are computed and not stored; k past n is
+    // masked on the A side; every wave computes all TPW tiles -- no branch may stand
+    // between MFMAs: the compiler was seen to leave out the wait for a result that is
+    // read on the far side of a taken branch)
+    __device__ __forceinline__ void product(const T *A, const T (&b)[NCB][CPW], v4 (&acc)[TPW]) const
+    {
+        const int lr = opaque(this->lr), lk = opaque(this->lk);
+        int row[TPW];
+#pragma unroll
+        for (int s = 0; s < TPW; s++) row[s] = min(rt(s) * 16 + lr, n - 1);
+        // (one k-step of operands ahead: all of them would fill the registers)
+        T a[TPW], an[TPW];
+        auto load_a = [&](int ks, T (&v)[TPW]) {
+            const int k = 4 * ks + lk, kc = min(k, n - 1);
+#pragma unroll
+            for (int s = 0; s < TPW; s++) v[s] = A[row[s] + n * kc];
+        };
+        load_a(0, a);
+#pragma unroll
+        for (int ks = 0; ks < CPW; ks++) {
+            if (ks + 1 < CPW) load_a(ks + 1, an);
+#pragma unroll
+            for (int s = 0; s < TPW; s++) acc[s] = M::run(4 * ks + lk < n ? a[s] : (T)0, b[cb(s)][ks], acc[s]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < TPW; s++) a[s] = an[s];
+        }
+    }
+    // f(tile s, element v, offset in a block) for every entry of the wave's tiles
+    template <class F>
+    __device__ __forceinline__ void each(F f) const
+    {
+        const int lr = opaque(this->lr), lk = opaque(this->lk);
+#pragma unroll
+        for (int s = 0; s < TPW; s++)
+            if (has(s))
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int i = rt(s) * 16 + M::row(lk, v), j = ct(cb(s)) * 16 + lr;
+                    if (i < n && j < n) f(s, v, i + n * j);
+                }
+    }
+};
+
+// dst[i] = src[i] for i < n by the workgroup, eight loads in flight per thread.
+template <typename T>
+__device__ __forceinline__ void wg_load_block_coh(T *dst, const T *src, long n)
+{
+    const int tid = threadIdx.x, nth = blockDim.x;
+    for (long b = tid; b < n; b += 8L * nth) {
+        T v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = coh_load(src, (int)min(b + (long)j * nth, n - 1));
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            if (b + (long)j * nth < n) dst[b + (long)j * nth] = v[j];
+    }
+}
+
+template <typename T>
+__host__ __device__ constexpr size_t factor_lds(int bsz)
+{
+    return ((size_t)3 * bsz * bsz * sizeof(T) + 15) / 16 * 16 + InvShared<T>::bytes(bsz);
+}
+
+// The row of ticket t, by the whole workgroup (a barrier must lie between two calls).
+// T: the factors' type (double, or float: the reference's single-precision
+// preconditioner, precPrecision 0, preprocessing/initializestructs.cpp:476-486, on the
+// FP32 MFMA).  Shared by the one-launch (WAIT) and level-launched kernels: the same bits.
+template <typename T, int RCH, int CPW, bool WAIT>
+__device__ __forceinline__ void factor_row(int n, const int *__restrict__ rowpts, const int *__restrict__ colind,
+                                           const int *__restrict__ u2o, const RowSched &sch, int t, T *Mg,
+                                           int *__restrict__ info, T *lds, const unsigned *flags, unsigned epoch,
+                                           int spin_limit, int *err)
+{
+    typedef BlockTiles<T, CPW> Tiles;
+    typedef typename Tiles::v4 v4;
+    constexpr int TPW = Tiles::TPW, NCB = Tiles::NCB;
+    const Tiles tl(n);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const long b2 = (long)n * n;
+    T *A = lds, *L = lds + b2, *Dg = lds + 2 * b2;
+    const InvShared<T> sh((char *)lds + ((size_t)3 * n * n * sizeof(T) + 15) / 16 * 16, n);
+    const int4 h = sch.rows[t];
+    const int ri = __builtin_amdgcn_readfirstlane(h.x), d0 = __builtin_amdgcn_readfirstlane(h.y);
+    const int first = __builtin_amdgcn_readfirstlane(h.z), cnt = __builtin_amdgcn_readfirstlane(h.w);
+    const int len = __builtin_amdgcn_readfirstlane(rowpts[ri + 1]) - d0;
+    if (len > FACTOR_MAXROW) {
+        // reported through info, the row is left as it is
+        if (tid == 0) info[ri] = -len;
+        return;
+    }
+    // lane l: column and number of the row's block l
+    const int rcol = lane < len ? colind[d0 + lane] : -1, rord = lane < len ? u2o[rcol] : -1;
+    const bool act = tl.active();
+    T *Mii = Mg + (long)d0 * b2;
+    wg_load_block_coh(Dg, (const T *)Mii, b2);
+    constexpr int NT = Tiles::NT;
+    // target block M_il -= L_ik U_kl (-L in LDS), tile column ct of it
+    auto update_target = [&](T *Mil, const T *U, int ct) {
+        const int lr = opaque(tl.lr), lk = opaque(tl.lk), j = ct * 16 + lr, jc = min(j, n - 1);
+        T b[CPW];
+        v4 c[NT];
+#pragma unroll
+        for (int ks = 0; ks < CPW; ks++) b[ks] = coh_load(U, min(4 * ks + lk, n - 1) + n * jc);
+#pragma unroll
+        for (int s = 0; s < NT; s++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                c[s][v] = coh_load((const T *)Mil, min(s * 16 + Tiles::M::row(lk, v), n - 1) + n * jc);
+        T a[NT], an[NT];
+        auto load_a = [&](int ks, T (&x)[NT]) {
+            const int kc = min(4 * ks + lk, n - 1);
+#pragma unroll
+            for (int s = 0; s < NT; s++) x[s] = L[min(s * 16 + lr, n - 1) + n * kc];
+        };
+        load_a(0, a);
+#pragma unroll
+        for (int ks = 0; ks < CPW; ks++) {
+            if (ks + 1 < CPW) load_a(ks + 1, an);
+#pragma unroll
+            for (int s = 0; s < NT; s++) c[s] = Tiles::M::run(4 * ks + lk < n ? a[s] : (T)0, b[ks], c[s]);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int s = 0; s < NT; s++) a[s] = an[s];
+        }
+#pragma unroll
+        for (int s = 0; s < NT; s++)
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                const int i = s * 16 + Tiles::M::row(lk, v);
+                if (i < n && j < n) coh_store(Mil, i + n * j, (T)c[s][v]);
+            }
+    };
+    // the targets left of the current neighbour: those of the last one are updated next to
+    // the inverse of the diagonal block, by waves 1-3
+    unsigned long long todo = 0;
+    int k0 = 0, km = -1, ct = 0, l = -1, w0 = 0;
+    // the wave's next (target, tile column): they are dealt to the waves, ct counts tile
+    // columns past the first of target l
+    auto pair = [&]() -> bool {
+        while (l < 0 || ct >= NT) {
+            if (!todo) return false;
+            if (l >= 0) ct -= NT;
+            l = __ffsll((long long)todo) - 1;
+            todo &= todo - 1;
+        }
+        update_target(Mg + (long)(d0 + l) * b2, Mg + (long)(k0 + __builtin_amdgcn_readlane(km, l)) * b2, ct);
+        ct += 4 - w0;
+        return true;
+    };
+    for (int q = 0; q < cnt; q++) {
+        const int2 e = sch.nbr[first + q];
+        T *Mik = Mg + (long)__builtin_amdgcn_readfirstlane(e.x) * b2;
+        const int rk = __builtin_amdgcn_readfirstlane(e.y);
+        k0 = __builtin_amdgcn_readfirstlane(rowpts[rk]);
+        const int klen = min(__builtin_amdgcn_readfirstlane(rowpts[rk + 1]) - k0, FACTOR_MAXROW);
+        const int ork = __builtin_amdgcn_readfirstlane(u2o[rk]);
+        const int ncol = lane < klen ? colind[k0 + lane] : -2;
+        // the previous neighbour's updates of A_ik are complete, and A, L free
+        if (q > 0) {
+            __builtin_amdgcn_s_waitcnt(0x0F70);   // s_waitcnt vmcnt(0)
+            __syncthreads();
+        }
+        wg_load_block_coh(A, (const T *)Mik, b2);
+        // lane l: position of the row's column l in row k, and the mask of targets
+        km = -1;
+        for (int m = 1; m < klen; m++) km = __builtin_amdgcn_readlane(ncol, m) == rcol ? m : km;
+        todo = __ballot(lane < len && km > 0 && (lane == 0 || rord > ork));
+        __syncthreads();
+        if (WAIT) wait_ready(flags + rk, epoch, spin_limit, err);
+        const bool diag = todo & 1;
+        const T *Mki = Mg + (long)(k0 + (diag ? __builtin_amdgcn_readlane(km, 0) : 0)) * b2;   // U_ki
+        todo &= ~1ull;
+        T bd[NCB][CPW];
+        if (act) {
+            T bi[NCB][CPW];
+            tl.load_b((const T *)Mg + (long)k0 * b2, bi);               // inv(U_kk)
+            if (diag && NCB == 1) tl.load_b(Mki, bd);                   // (two tile columns of both do not fit)
+            v4 lc[TPW];
+#pragma unroll
+            for (int s = 0; s < TPW; s++) lc[s] = (v4){(T)0, (T)0, (T)0, (T)0};
+            tl.product(A, bi, lc);
+            tl.each([&](int s, int v, int o) {
+                L[o] = -lc[s][v];
+                *entry(Mik, o) = lc[s][v];
+            });
+            if (diag && NCB > 1) tl.load_b(Mki, bd);
+        }
+        __syncthreads();
+        if (act && diag) {
+            v4 dg[TPW];
+            tl.each([&](int s, int v, int o) { dg[s][v] = Dg[o]; });
+            tl.product(L, bd, dg);
+            tl.each([&](int s, int v, int o) { Dg[o] = dg[s][v]; });
+        }
+        w0 = q + 1 == cnt;
+        ct = tl.wv - w0;
+        l = -1;
+        if (!w0)
+            while (pair()) {}
+    }
+    __syncthreads();
+    const int r = wg_inverse<T, NT>(n, Dg, sh, [&] { pair(); }, [&](int i, int c, T v) { coh_store(Mii, i + n * c, v); });
+    if (tl.wv > 0)
+        while (pair()) {}
+    if (tid == 0) info[ri] = r;
+}
+
+// The rows of one level: tickets [t0, t1).
+template <typename T, int RCH, int CPW>
+__global__ void __launch_bounds__(SV_THREADS, RCH == 1 ? 2 : 1)
+bilu0_factor_kernel(int bsz, const int *__restrict__ rowpts, const int *__restrict__ colind,
+                    const int *__restrict__ u2o, RowSched sch, int t0, int t1, T *Mg, int *__restrict__ info)
+{
+    extern __shared__ __align__(16) double lds_raw[];
+    for (int t = t0 + blockIdx.x; t < t1; t += gridDim.x) {
+        factor_row<T, RCH, CPW, false>(bsz, rowpts, colind, u2o, sch, t, Mg, info, (T *)lds_raw, nullptr, 0, 0, nullptr);
+        __syncthreads();
+    }
+}
+
+// The whole factorisation in one launch: the rows in ticket order (the forward levels
+// concatenated) to persistent workgroups through an atomic ticket, as in
+// bilu0_sweep_syncfree_kernel.  Before reading row k's blocks every wave waits for k's
+// ready flag, which holds the launch's epoch once all of k's blocks are final.  A row
+// too long for the factorisation is reported through info and still published.
+template <typename T, int RCH, int CPW>
+__global__ void __launch_bounds__(SV_THREADS, RCH == 1 ? 2 : 1)
+bilu0_factor_syncfree_kernel(int bsz, const int *__restrict__ rowpts, const int *__restrict__ colind,
+                             const int *__restrict__ u2o, RowSched sch, int n, T *Mg, int *__restrict__ info,
+                             unsigned *flags, const unsigned *epoch_p, unsigned *counter, int spin_limit, int *err)
+{
+    extern __shared__ __align__(16) double lds_raw[];
+    __shared__ int sticket;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const unsigned epoch = __hip_atomic_load(epoch_p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // (loop control wave-uniform throughout: see bilu0_sweep_syncfree_kernel)
+    while (true) {
+        if (wv == 0) sticket = __builtin_amdgcn_readfirstlane(atomicAdd(counter, lane == 0 ? 1u : 0u));
+        __syncthreads();
+        const int t = __builtin_amdgcn_readfirstlane(sticket);
+        if (t >= n) break;
+        factor_row<T, RCH, CPW, true>(bsz, rowpts, colind, u2o, sch, t, Mg, info, (T *)lds_raw, flags, epoch,
+                                      spin_limit, err);
+        // publish the row once every wave's stores of it have completed (vmcnt 0:
+        // device-scope stores are acknowledged at the coherence point)
+        __builtin_amdgcn_s_waitcnt(0x0F70);   // s_waitcnt vmcnt(0)
+        __syncthreads();
+        if (wv == 0)
+            __hip_atomic_store(flags + __builtin_amdgcn_readfirstlane(sch.rows[t].x), epoch, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
 // A new epoch for the factorisation's ready flags (so that they are never cleared)
 // and a fresh ticket.
 __global__ void factor_reset_kernel(unsigned *sync)
@@ -758,146 +959,6 @@ __global__ void factor_reset_kernel(unsigned *sync)
         unsigned e = sync[0] + 1;
         sync[0] = e == 0 ? 1 : e;
         sync[1] = 0;
-    }
-}
-
-// Block copy and subtraction through agent-scope atomics (coherent across the
-// XCDs), with the entry -> thread map of wg_load_block / wg_subtract_block: the
-// sync-free factorisation reads and writes the factor blocks only this way, since
-// rows are factored by workgroups on any XCD.
-template <typename T>
-__device__ __forceinline__ void wg_load_block_coh(T *dst, const T *src, long n)
-{
-    const int tid = threadIdx.x, nth = blockDim.x;
-    for (long b = tid; b < n; b += 8L * nth) {
-        T v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            v[j] = __hip_atomic_load(src + min(b + (long)j * nth, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (b + (long)j * nth < n) dst[b + (long)j * nth] = v[j];
-    }
-}
-
-template <typename T>
-__device__ __forceinline__ void wg_subtract_block_coh(T *dst, const T *d, long n)
-{
-    const int tid = threadIdx.x, nth = blockDim.x;
-    for (long b = tid; b < n; b += 8L * nth) {
-        T v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            v[j] = __hip_atomic_load(dst + min(b + (long)j * nth, n - 1), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-        for (int j = 0; j < 8; j++)
-            if (b + (long)j * nth < n)
-                __hip_atomic_store(dst + b + (long)j * nth, v[j] - d[b + (long)j * nth], __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-    }
-}
-
-// The BILU0 factorisation without level launches: bilu0_factor_kernel's per-row
-// arithmetic (the same bits) with the rows taken in `order` (the level lists
-// concatenated) by persistent workgroups through an atomic ticket, as in
-// bilu0_sweep_syncfree_kernel.  Before reading row k's blocks (inv(U_kk) and U_kl)
-// every wave waits for k's ready flag, set once all of k's blocks are final; the
-// blocks go through agent-scope atomics (wg_load_block_coh / wg_subtract_block_coh)
-// and the flag is stored after every wave's stores have completed.  A row too long
-// for the factorisation is reported through info and still published.
-template <typename T>
-__global__ void __launch_bounds__(SV_THREADS)
-bilu0_factor_syncfree_kernel(int bsz, const int *__restrict__ rowpts, const int *__restrict__ colind,
-                             const int *__restrict__ u2o, const int *__restrict__ order, int n, T *Mg,
-                             int *__restrict__ info, unsigned *flags, const unsigned *epoch_p, unsigned *counter,
-                             int spin_limit, int *err)
-{
-    extern __shared__ double lds_raw[];
-    T *lds = (T *)lds_raw;
-    const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const long b2 = (long)bsz * bsz;
-    T *X = lds, *B = lds + b2, *L = lds + 2 * b2;
-    LdsInv<T> w = lds_inv_area(lds + 3 * b2, bsz);
-    int *rcol = w.piv + bsz + 2, *rord = rcol + FACTOR_MAXROW, *lst = rord + FACTOR_MAXROW,
-        *ncol = lst + FACTOR_MAXROW + 1, *sticket = ncol + FACTOR_MAXROW;
-    const unsigned epoch = __hip_atomic_load(epoch_p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // (loop control wave-uniform throughout: see bilu0_sweep_syncfree_kernel)
-    while (true) {
-        if (wv == 0) *sticket = __builtin_amdgcn_readfirstlane(atomicAdd(counter, lane == 0 ? 1u : 0u));
-        __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(*sticket);
-        if (t >= n) break;
-        const int ri = order[t], oi = u2o[ri], d0 = rowpts[ri], len = rowpts[ri + 1] - d0;
-        if (len <= FACTOR_MAXROW) {
-            if (tid < len) {
-                const int c = colind[d0 + tid];
-                rcol[tid] = c;
-                rord[tid] = u2o[c];
-            }
-            __syncthreads();
-            if (tid == 0) {
-                int cnt = 0;
-                for (int q = 1; q < len; q++) {
-                    if (rord[q] >= oi) continue;
-                    int m = cnt++;
-                    while (m > 0 && rord[lst[1 + m - 1]] > rord[q]) {
-                        lst[1 + m] = lst[1 + m - 1];
-                        m--;
-                    }
-                    lst[1 + m] = q;
-                }
-                lst[0] = cnt;
-            }
-            __syncthreads();
-            const int cnt = __builtin_amdgcn_readfirstlane(lst[0]);
-            for (int qq = 0; qq < cnt; qq++) {
-                const int q = __builtin_amdgcn_readfirstlane(lst[1 + qq]);
-                const int ik = d0 + q, rk = __builtin_amdgcn_readfirstlane(rcol[q]);
-                const int ork = __builtin_amdgcn_readfirstlane(rord[q]);
-                const int k0 = rowpts[rk], klen = rowpts[rk + 1] - k0;
-                if (tid < klen && tid < FACTOR_MAXROW) ncol[tid] = colind[k0 + tid];
-                wait_ready(flags + rk, epoch, spin_limit, err);
-                wg_load_block_coh(X, Mg + (long)ik * b2, b2);
-                wg_load_block_coh(B, Mg + (long)k0 * b2, b2);     // inv(U_kk)
-                __syncthreads();
-                T *Mik = Mg + (long)ik * b2;
-                lds_block_product(X, B, bsz, [&](int i, int j, T c) {
-                    L[i + bsz * j] = c;
-                    __hip_atomic_store(Mik + i + bsz * j, c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                });
-                __syncthreads();
-                for (int l = 0; l < len; l++) {
-                    if (l != 0 && __builtin_amdgcn_readfirstlane(rord[l]) <= ork) continue;
-                    const int rl = __builtin_amdgcn_readfirstlane(rcol[l]);
-                    int km = -1;
-                    for (int m = 1; m < klen && m < FACTOR_MAXROW; m++)
-                        if (__builtin_amdgcn_readfirstlane(ncol[m]) == rl) {
-                            km = m;
-                            break;
-                        }
-                    if (km < 0) continue;
-                    wg_load_block_coh(B, Mg + (long)(k0 + km) * b2, b2);
-                    __syncthreads();
-                    lds_block_product(L, B, bsz, [&](int i, int j, T c) { X[i + bsz * j] = c; });
-                    __syncthreads();
-                    wg_subtract_block_coh(Mg + (long)(d0 + l) * b2, X, b2);
-                    __syncthreads();
-                }
-                __syncthreads();
-            }
-            wg_load_block_coh(X, Mg + (long)d0 * b2, b2);
-            __syncthreads();
-            const int r = lds_inverse(X, bsz, w.piv, w.rowk, w.colk, w.red);
-            for (long i = tid; i < b2; i += nth)
-                __hip_atomic_store(Mg + (long)d0 * b2 + i, X[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (tid == 0) info[ri] = r;
-        } else {
-            if (tid == 0) info[ri] = -len;
-        }
-        // publish row ri once every wave's stores of it have completed
-        __builtin_amdgcn_s_waitcnt(0x0F70);   // s_waitcnt vmcnt(0)
-        __syncthreads();
-        if (wv == 0) __hip_atomic_store(flags + ri, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
@@ -1043,20 +1104,25 @@ static hipError_t set_lds(const void *fn, size_t bytes)
     return hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
 }
 
-size_t block_inverse_lds(int bsz) { return sizeof(double) * bsz * bsz + lds_inv_bytes(bsz); }
-size_t bilu0_factor_lds(int bsz)
+size_t block_inverse_lds(int bsz)
 {
-    return sizeof(double) * 3 * bsz * bsz + lds_inv_bytes(bsz) + sizeof(int) * (4 * FACTOR_MAXROW + 1);
+    return sizeof(double) * (bsz * bsz + 1) / 16 * 16 + 16 + InvShared<double>::bytes(bsz);
 }
+// (no factorisation shape beyond a block size of 80)
+size_t bilu0_factor_lds(int bsz) { return bsz <= 80 ? factor_lds<double>(bsz) : ~(size_t)0 / 2; }
 
 hipError_t launch_block_inverse(int nrows, int bsz, const int *rowpts, const double *Hg, double *Dinv, int *info,
                                 hipStream_t s)
 {
     const size_t lds = block_inverse_lds(bsz);
-    hipError_t e = set_lds((const void *)block_inverse_kernel, lds);
+    if (bsz < 1 || bsz > 128) return hipErrorInvalidValue;
+    const int nt = (bsz + 15) / 16;
+    auto kernel = nt == 1 ? block_inverse_kernel<1> : nt == 2 ? block_inverse_kernel<2> : nt == 3 ? block_inverse_kernel<3>
+                : nt == 4 ? block_inverse_kernel<4> : nt == 5 ? block_inverse_kernel<5> : block_inverse_kernel<8>;
+    hipError_t e = set_lds((const void *)kernel, lds);
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(block_inverse_kernel, dim3(std::min(nrows, 8192)), dim3(SV_THREADS), lds, s, nrows, bsz,
-                       rowpts, Hg, Dinv, info);
+    hipLaunchKernelGGL(kernel, dim3(std::min(nrows, 8192)), dim3(SV_THREADS), lds, s, nrows, bsz, rowpts, Hg, Dinv,
+                       info);
     return hipGetLastError();
 }
 
@@ -1071,56 +1137,71 @@ hipError_t launch_mdf_weights(int nrows, int bsz, const int *rowpts, const doubl
     return hipGetLastError();
 }
 
-template <typename T>
-static hipError_t factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows, int nlev,
-                               T *Mg, int *info, hipStream_t s)
+// (block sizes above 80 have no factorisation shape: bilu0_factor_lds)
+template <class F>
+static hipError_t factor_shape(int bsz, F launch)
 {
-    const size_t lds = bilu0_factor_lds(bsz);
-    hipError_t e = set_lds((const void *)bilu0_factor_kernel<T>, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(bilu0_factor_kernel<T>, dim3(std::min(nlev, 8192)), dim3(SV_THREADS), lds, s, bsz, rowpts,
-                       colind, u2o, rows, nlev, Mg, info);
-    return hipGetLastError();
+    if (bsz > 80) return hipErrorInvalidValue;
+    return block_shape(bsz, [&](auto R, auto C) {
+        if constexpr (C() <= 20) launch(R, C);
+    });
 }
 
 template <typename T>
-static hipError_t factor_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *order, int n,
-                                  T *Mg, int *info, unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err,
-                                  hipStream_t s)
+static hipError_t factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const RowSched &sch,
+                               int t0, int t1, T *Mg, int *info, hipStream_t s)
+{
+    const size_t lds = factor_lds<T>(bsz);
+    return factor_shape(bsz, [&](auto R, auto C) {
+        if (set_lds((const void *)bilu0_factor_kernel<T, R(), C()>, lds) == hipSuccess)
+            hipLaunchKernelGGL((bilu0_factor_kernel<T, R(), C()>), dim3(std::min(t1 - t0, 8192)), dim3(SV_THREADS), lds,
+                               s, bsz, rowpts, colind, u2o, sch, t0, t1, Mg, info);
+    });
+}
+
+template <typename T>
+static hipError_t factor_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o, const RowSched &sch,
+                                  int n, T *Mg, int *info, unsigned *flags, unsigned *sync, int nwg, int spin_limit,
+                                  int *err, hipStream_t s)
 {
     if (n <= 0 || nwg <= 0) return hipErrorInvalidValue;
-    const size_t lds = bilu0_factor_lds(bsz) + 16;   // and the ticket
-    hipError_t e = set_lds((const void *)bilu0_factor_syncfree_kernel<T>, lds);
-    if (e != hipSuccess) return e;
+    const size_t lds = factor_lds<T>(bsz);
     hipLaunchKernelGGL(factor_reset_kernel, dim3(1), dim3(64), 0, s, sync);
-    hipLaunchKernelGGL(bilu0_factor_syncfree_kernel<T>, dim3(std::min(n, nwg)), dim3(SV_THREADS), lds, s, bsz, rowpts,
-                       colind, u2o, order, n, Mg, info, flags, sync, sync + 1, spin_limit, err);
-    return hipGetLastError();
+    return factor_shape(bsz, [&](auto R, auto C) {
+        if (set_lds((const void *)bilu0_factor_syncfree_kernel<T, R(), C()>, lds) == hipSuccess)
+            hipLaunchKernelGGL((bilu0_factor_syncfree_kernel<T, R(), C()>), dim3(std::min(n, nwg)), dim3(SV_THREADS),
+                               lds, s, bsz, rowpts, colind, u2o, sch, n, Mg, info, flags, sync, sync + 1, spin_limit,
+                               err);
+    });
 }
 
 hipError_t launch_bilu0_factor_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o,
-                                        const int *order, int n, double *Mg, int *info, unsigned *flags,
-                                        unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s)
+                                        const int4 *rows, const int2 *nbr, int n, double *Mg, int *info,
+                                        unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err,
+                                        hipStream_t s)
 {
-    return factor_syncfree(bsz, rowpts, colind, u2o, order, n, Mg, info, flags, sync, nwg, spin_limit, err, s);
+    return factor_syncfree(bsz, rowpts, colind, u2o, RowSched{rows, nbr}, n, Mg, info, flags, sync, nwg, spin_limit,
+                           err, s);
 }
 hipError_t launch_bilu0_factor_syncfree(int bsz, const int *rowpts, const int *colind, const int *u2o,
-                                        const int *order, int n, float *Mg, int *info, unsigned *flags,
-                                        unsigned *sync, int nwg, int spin_limit, int *err, hipStream_t s)
+                                        const int4 *rows, const int2 *nbr, int n, float *Mg, int *info,
+                                        unsigned *flags, unsigned *sync, int nwg, int spin_limit, int *err,
+                                        hipStream_t s)
 {
-    return factor_syncfree(bsz, rowpts, colind, u2o, order, n, Mg, info, flags, sync, nwg, spin_limit, err, s);
+    return factor_syncfree(bsz, rowpts, colind, u2o, RowSched{rows, nbr}, n, Mg, info, flags, sync, nwg, spin_limit,
+                           err, s);
 }
 
-hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, double *Mg, int *info, hipStream_t s)
+hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int4 *rows,
+                                     const int2 *nbr, int t0, int t1, double *Mg, int *info, hipStream_t s)
 {
-    return factor_level(bsz, rowpts, colind, u2o, rows, nlev, Mg, info, s);
+    return factor_level(bsz, rowpts, colind, u2o, RowSched{rows, nbr}, t0, t1, Mg, info, s);
 }
 
-hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int *rows,
-                                     int nlev, float *Mg, int *info, hipStream_t s)
+hipError_t launch_bilu0_factor_level(int bsz, const int *rowpts, const int *colind, const int *u2o, const int4 *rows,
+                                     const int2 *nbr, int t0, int t1, float *Mg, int *info, hipStream_t s)
 {
-    return factor_level(bsz, rowpts, colind, u2o, rows, nlev, Mg, info, s);
+    return factor_level(bsz, rowpts, colind, u2o, RowSched{rows, nbr}, t0, t1, Mg, info, s);
 }
 
 template <typename TM>
@@ -1146,36 +1227,17 @@ hipError_t launch_bilu0_scale_upper(int bsz, int n, const int *rowpts, const int
     return scale_upper(bsz, n, rowpts, colind, u2o, Mg, s);
 }
 
-// The sweep kernels' shapes by block size: CPW columns per wave, NPRE neighbours'
-// shares in registers (up to about 128 VGPRs of them).  A shape's unused columns cost
-// their loads, so the sizes in use have one that fits: 8-16 (triangles p=1-3), 20 and
-// 24 (p=4, 5, hexes p=1), 30 (tets p=2), 45 (hexes p=2), 50 (tets p=3); 75 (tets p=4)
-// and above take two rows per lane.
-template <class F>
-static hipError_t sweep_shape(int bsz, F launch)
-{
-    using std::integral_constant;
-#define SHAPE(R, C, P) \
-    launch(integral_constant<int, R>(), integral_constant<int, C>(), integral_constant<int, P>())
-    if (bsz < 1 || bsz > 128) return hipErrorInvalidValue;
-    if (bsz <= 16) SHAPE(1, 4, 8);
-    else if (bsz <= 24) SHAPE(1, 6, 8);
-    else if (bsz <= 32) SHAPE(1, 8, 6);
-    else if (bsz <= 48) SHAPE(1, 12, 5);
-    else if (bsz <= 52) SHAPE(1, 13, 4);
-    else if (bsz <= 64) SHAPE(1, 16, 4);
-    else if (bsz <= 80) SHAPE(2, 20, 1);
-    else SHAPE(2, 32, 1);
-#undef SHAPE
-    return hipGetLastError();
-}
+// Neighbours' shares a sweep keeps in registers (up to about 128 VGPRs of them; the
+// sweeps' times hardly change between 2 and 4 at 50 columns).
+constexpr int sweep_ahead(int rch, int cpw) { return rch > 1 ? 1 : cpw <= 6 ? 8 : cpw <= 8 ? 6 : cpw <= 12 ? 5 : 4; }
 
 template <bool BACKWARD, typename TM>
 static hipError_t sweep_level(int bsz, const RowSched &sch, int t0, int t1, const TM *Mg, const double *x, double *y,
                               hipStream_t s)
 {
-    return sweep_shape(bsz, [&](auto R, auto C, auto P) {
-        hipLaunchKernelGGL((bilu0_sweep_kernel<BACKWARD, R(), C(), P(), TM>), dim3(std::min(t1 - t0, 8192)),
+    return block_shape(bsz, [&](auto R, auto C) {
+        constexpr int P = sweep_ahead(R(), C());
+        hipLaunchKernelGGL((bilu0_sweep_kernel<BACKWARD, R(), C(), P, TM>), dim3(std::min(t1 - t0, 8192)),
                            dim3(SV_THREADS), 0, s, bsz, sch, t0, t1, Mg, x, y);
     });
 }
@@ -1212,10 +1274,11 @@ static hipError_t sweeps_syncfree(int bsz, const RowSched &low, const RowSched &
     const int g = std::min(n, nwg);
     const long N = (long)n * bsz;
     hipLaunchKernelGGL(sweep_reset_kernel, dim3(grid_for(N)), dim3(SV_THREADS), 0, s, sync, N, t, y);
-    return sweep_shape(bsz, [&](auto R, auto C, auto P) {
-        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<false, R(), C(), P(), TM>), dim3(g), dim3(SV_THREADS), 0, s,
+    return block_shape(bsz, [&](auto R, auto C) {
+        constexpr int P = sweep_ahead(R(), C());
+        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<false, R(), C(), P, TM>), dim3(g), dim3(SV_THREADS), 0, s,
                            bsz, low, n, Mg, x, t, sync + 1, spin_limit, err);
-        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<true, R(), C(), P(), TM>), dim3(g), dim3(SV_THREADS), 0, s,
+        hipLaunchKernelGGL((bilu0_sweep_syncfree_kernel<true, R(), C(), P, TM>), dim3(g), dim3(SV_THREADS), 0, s,
                            bsz, up, n, Mg, t, y, sync + 2, spin_limit, err);
     });
 }
