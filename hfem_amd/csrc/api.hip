@@ -123,7 +123,7 @@ extern "C" int hfem_destroy(hfem_ctx *c)
                     c->rowstart, c->cols, c->einv, c->f2e, c->blkptr, c->blklist, c->UDG, c->UH, c->SH, c->D, c->Fx,
                     c->X, c->K, c->Hx, c->Ru, c->Rh, c->ru2, c->info, c->dinv, c->spill, c->rwork, c->fluxbuf, c->Hg, c->Rg,
                     c->r, c->partial, c->xv, c->yv, c->sv.d_u2o, c->sv.d_lsched, c->sv.d_usched,
-                    c->sv.d_lnbr, c->sv.d_unbr,
+                    c->sv.d_lnbr, c->sv.d_unbr, c->sv.d_fnbr,
                     c->sv.Mg, c->sv.Mg32, c->sv.gy, c->sv.Dinv, c->sv.Cw, c->sv.d_info, c->sv.x, c->sv.V, c->sv.b, c->sv.t, c->sv.dots,
                     c->sv.coef, c->sv.UDGi, c->sv.sf_flags, c->sv.sf_err, c->qn_dinv, c->qn_K, c->rdmax, c->rcmax, c->rdprev, c->rcount};
     for (void *p : ptrs)

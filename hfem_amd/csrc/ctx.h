@@ -153,7 +153,7 @@ struct SolverState {
     bool sched_valid = false;           // the device copies below are the current ordering's
     // the sweeps' rows in level order with their neighbours (RowSched, solver.hip)
     int4 *d_lsched = nullptr, *d_usched = nullptr;
-    int2 *d_lnbr = nullptr, *d_unbr = nullptr;
+    int2 *d_lnbr = nullptr, *d_unbr = nullptr, *d_fnbr = nullptr;
     double *Mg = nullptr;               // BILU0 factors (nblocks blocks) or block-Jacobi inverses (nf blocks)
     float *Mg32 = nullptr;              // the same in single precision (precPrecision 0)
     int prec_fp32 = 0;

@@ -88,7 +88,7 @@ struct InvShared {
 // All threads call it with the block complete (a barrier before); out(i, c, v) receives
 // every entry of the inverse once, rows along the lanes.  Returns 0, or 1 + the step of
 // the first zero pivot (workgroup-uniform; the result is then finite but no inverse).
-template <typename T, int NT, class IDLE, class OUT>
+template <int NT, class IDLE, class OUT, typename T>
 __device__ __forceinline__ int wg_inverse(int n, T *A, const InvShared<T> &sh, IDLE idle, OUT out)
 {
     typedef BlkMfma<T> M;
@@ -216,6 +216,290 @@ __device__ __forceinline__ int wg_inverse(int n, T *A, const InvShared<T> &sh, I
     return __builtin_amdgcn_readfirstlane(*sh.sing);
 }
 
+// ---- inverse of one block, entry by entry ----
+//
+// The inverse of the single-precision BILU0 factors: the same waves, panels and barriers,
+// but every entry goes through the plain elimination's operations one by one,
+// a - c (r pinv), on the vector ALU.  Along the rows of a factorisation roundings can
+// grow: on 4 608 p=4 triangles (849 levels) those of single precision reach 3e-3 to 5e-3
+// of M^-1 x, and the order of the sums alone moved a Newton iterate by 1e-6; this form's
+// roundings are those of the unblocked elimination.  (Pivots, ties included, are chosen as
+// if the rows were interchanged: pos is the place of a row.)
+// The factorisation of those triangles: 13.1 ms (10.1 with the blocked inverse, 34.1 with
+// the block in LDS and a barrier around every pass), of the 8^3 p=2 hexes 13.4 (9.6, 37.5).
+template <typename T> struct StepShared;
+template <>
+struct StepShared<float> {
+    static constexpr int bytes(int rows) { return (2 * 16 * rows + 2 * 16) * 4 + (2 * 16 + 2 * rows + 1) * 4; }
+    float *c, *pinv;                 // per panel's parity: 16 pivot columns (0 in the pivot row), 16 reciprocals
+    int *prow, *lab, *pof, *sing;    // per panel's parity: the pivot rows; per row its step; per step its row
+    __device__ StepShared(void *mem, int rows)
+    {
+        c = (float *)mem;
+        pinv = c + 2 * 16 * rows;
+        prow = (int *)(pinv + 2 * 16);
+        lab = prow + 2 * 16;
+        pof = lab + rows;
+        sing = pof + rows;
+    }
+};
+
+// Entry `row` (wave-uniform) of a column held with rows lane + 64 q.
+template <int RPL>
+__device__ __forceinline__ float row_bcast(const float (&col)[RPL], int row)
+{
+    if constexpr (RPL == 1) return GJ<float>::bcast(col[0], row);
+    else return GJ<float>::bcast(row < 64 ? col[0] : col[1], row & 63);
+}
+
+// The pivot steps k0 ... k0 + kw - 1 of a panel on one wave (rows lane + 64 q; the columns
+// rotate through x: column k is left in x[16 - kw + k]).  Stores step k's pivot column to
+// c[n k ...]; lane k returns its pivot row in prow, its reciprocal in pinvs.
+template <int RPL>
+struct PivotSteps {
+    unsigned open[RPL];
+    int pos[RPL], lab[RPL], sing;
+    __device__ __forceinline__ void init(int n)
+    {
+        sing = 0;
+#pragma unroll
+        for (int q = 0; q < RPL; q++) {
+            pos[q] = (threadIdx.x & 63) + 64 * q;
+            open[q] = pos[q] < n ? ~0u : 0u;
+            lab[q] = -1;
+        }
+    }
+    __device__ __forceinline__ void run(float (&x)[16][RPL], int kw, int k0, int n, float *c, int &prow, float &pinvs)
+    {
+        const int lane = threadIdx.x & 63;
+        unsigned key[RPL], m = 0;
+        int p = 0;
+        float pv = 0.0f, pinv = 0.0f, row1 = 0.0f;
+        prow = 0;
+        pinvs = 1.0f;
+        auto search = [&](int stage, const float (&col)[RPL], const float (&next)[RPL]) {
+            switch (stage) {
+            case 0:
+#pragma unroll
+                for (int q = 0; q < RPL; q++) key[q] = pivot_key(col[q]) & open[q];
+                m = key[0];
+#pragma unroll
+                for (int q = 1; q < RPL; q++) m = max(m, key[q]);
+                m = key_max_step<0>(m);
+                break;
+            case 1: m = key_max_step<1>(m); m = key_max_step<2>(m); break;
+            case 2: m = key_max_step<3>(m); m = key_max_step<4>(m); break;
+            case 3: m = key_max_step<5>(m); break;
+            case 4: {
+                const unsigned mm = (unsigned)__builtin_amdgcn_readlane((int)m, 63);
+                int ties = 0;
+#pragma unroll
+                for (int q = RPL - 1; q >= 0; q--) {
+                    const unsigned long long b = __ballot(key[q] == mm);
+                    p = b ? 64 * q + __ffsll((long long)b) - 1 : p;
+                    ties += __popcll(b);
+                }
+                if (ties > 1) {
+                    // the first in place (128 - pos > 0)
+                    unsigned t[RPL], best = 0;
+#pragma unroll
+                    for (int q = 0; q < RPL; q++) {
+                        t[q] = key[q] == mm ? 128u - (unsigned)pos[q] : 0u;
+                        best = max(best, t[q]);
+                    }
+                    best = wave_max_key(best);
+#pragma unroll
+                    for (int q = 0; q < RPL; q++) {
+                        const unsigned long long b = __ballot(t[q] == best);
+                        p = b ? 64 * q + __ffsll((long long)b) - 1 : p;
+                    }
+                }
+                break;
+            }
+            case 5:
+                pv = row_bcast<RPL>(col, p);
+                row1 = row_bcast<RPL>(next, p);
+                break;
+            case 6: pinv = pv == 0.0f ? 0.0f : 1.0f / pv; break;
+            }
+        };
+        constexpr int NS = 7;
+#pragma unroll
+        for (int st = 0; st < NS; st++) search(st, x[0], x[1]);
+#pragma unroll 1
+        for (int k = 0; k < kw; k++) {
+            bool mine[RPL];
+            float cz[RPL], f[RPL], last[RPL];
+            const float s1 = row1 * pinv;
+            const int posp = RPL == 1 || p < 64 ? __builtin_amdgcn_readlane(pos[0], p & 63)
+                                                : __builtin_amdgcn_readlane(pos[RPL - 1], p & 63);
+#pragma unroll
+            for (int q = 0; q < RPL; q++) {
+                mine[q] = lane + 64 * q == p;
+                cz[q] = mine[q] ? 0.0f : x[0][q];
+                f[q] = mine[q] ? pinv : 1.0f;
+                last[q] = mine[q] ? pinv : -x[0][q] * pinv;
+                x[0][q] = mine[q] ? s1 : fmaf(-cz[q], s1, x[1][q]);
+                open[q] = mine[q] ? 0u : open[q];
+            }
+            const int pk = p;
+            const float pinvk = pinv;
+            const bool zero = pv == 0.0f;
+            // (after the last step: of a column that is none, unused)
+#pragma unroll
+            for (int st = 0; st < NS; st++) {
+                // columns 2-15: st = 0 ... 6 takes two each, column 2 (the next step's second)
+                // first
+                search(st, x[0], x[1]);
+                __builtin_amdgcn_sched_barrier(0);
+                if (st == 0) {
+#pragma unroll
+                    for (int q = 0; q < RPL; q++) {
+                        pos[q] = mine[q] ? k0 + k : pos[q] == k0 + k ? posp : pos[q];
+                        lab[q] = mine[q] ? k0 + k : lab[q];
+                        if (lane + 64 * q < n) c[n * k + lane + 64 * q] = cz[q];
+                    }
+                    sing = zero && !sing ? k0 + k + 1 : sing;
+                    prow = lane == k ? pk : prow;
+                    pinvs = lane == k ? pinvk : pinvs;
+                }
+#pragma unroll
+                for (int j = 2 + 2 * st; j < 4 + 2 * st; j++) {
+                    float y[RPL];
+#pragma unroll
+                    for (int q = 0; q < RPL; q++) y[q] = x[j][q] * f[q];
+                    const float sj = row_bcast<RPL>(y, pk);
+#pragma unroll
+                    for (int q = 0; q < RPL; q++) x[j - 1][q] = fmaf(-cz[q], sj, y[q]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int q = 0; q < RPL; q++) x[15][q] = last[q];
+        }
+    }
+};
+
+// As wg_inverse.
+template <int NT, class IDLE, class OUT>
+__device__ __forceinline__ int wg_inverse(int n, float *A, const StepShared<float> &sh, IDLE idle, OUT out)
+{
+    constexpr int RPL = NT <= 4 ? 1 : 2;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int np = (n + 15) / 16, ng = (n + 3) / 4;
+    PivotSteps<RPL> ps;
+    if (wv == 0) ps.init(n);
+    // panel pb's steps on columns 4 g ... 4 g + 3
+    auto update = [&](int pb, int g) {
+        const int kw = min(16, n - 16 * pb);
+        const float *c = sh.c + (pb & 1) * 16 * n;
+        float x[4][RPL], cn[RPL];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int q = 0; q < RPL; q++) x[u][q] = A[min(lane + 64 * q, n - 1) + n * min(4 * g + u, n - 1)];
+#pragma unroll
+        for (int q = 0; q < RPL; q++) cn[q] = c[min(lane + 64 * q, n - 1)];
+        const int pr = sh.prow[(pb & 1) * 16 + (lane & 15)];
+        const float pi = sh.pinv[(pb & 1) * 16 + (lane & 15)];
+#pragma unroll 2
+        for (int k = 0; k < kw; k++) {
+            const int p = __builtin_amdgcn_readlane(pr, k);
+            const float pinv = GJ<float>::bcast(pi, k);
+            float ck[RPL], f[RPL];
+#pragma unroll
+            for (int q = 0; q < RPL; q++) {
+                ck[q] = cn[q];
+                f[q] = lane + 64 * q == p ? pinv : 1.0f;
+                cn[q] = c[min(lane + 64 * q, n - 1) + n * min(k + 1, kw - 1)];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                float y[RPL];
+#pragma unroll
+                for (int q = 0; q < RPL; q++) y[q] = x[u][q] * f[q];
+                const float s = row_bcast<RPL>(y, p);
+#pragma unroll
+                for (int q = 0; q < RPL; q++) x[u][q] = fmaf(-ck[q], s, y[q]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int q = 0; q < RPL; q++)
+                if (4 * g + u < n && lane + 64 * q < n) A[lane + 64 * q + n * (4 * g + u)] = x[u][q];
+    };
+    for (int pb = 0;; pb++) {
+        if (pb > 0 && pb < np) {
+            // the next panel's columns over all four waves
+            if (4 * pb + wv < ng) update(pb - 1, 4 * pb + wv);
+            __syncthreads();
+        }
+        // the other columns over waves 1-3 (after the last panel over all four)
+        for (int g = 0, d = pb < np; pb > 0 && g < ng; g++) {
+            if (g >> 2 == pb - 1 || g >> 2 == pb) continue;
+            if (wv == d) update(pb - 1, g);
+            d = d == 3 ? pb < np : d + 1;
+        }
+        if (pb == np) break;
+        if (wv == 0) {
+            const int kw = min(16, n - 16 * pb);
+            float x[16][RPL], pinvs;
+            int prow;
+#pragma unroll
+            for (int j = 0; j < 16; j++)
+#pragma unroll
+                for (int q = 0; q < RPL; q++) x[j][q] = A[min(lane + 64 * q, n - 1) + n * min(16 * pb + j, n - 1)];
+            ps.run(x, kw, 16 * pb, n, sh.c + (pb & 1) * 16 * n, prow, pinvs);
+            float *P = A + n * (16 * pb + kw - 16);
+#pragma unroll
+            for (int q = 0; q < RPL; q++)
+                if (lane + 64 * q < n) {
+#pragma unroll
+                    for (int j = 0; j < 16; j++)
+                        if (j >= 16 - kw) P[lane + 64 * q + n * j] = x[j][q];
+                    sh.lab[lane + 64 * q] = ps.lab[q];
+                }
+            if (lane < kw) {
+                sh.prow[(pb & 1) * 16 + lane] = prow;
+                sh.pinv[(pb & 1) * 16 + lane] = pinvs;
+                sh.pof[16 * pb + lane] = prow;
+            }
+            if (lane == 0) *sh.sing = ps.sing;
+        } else {
+            idle();
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    int lab[RPL], pof[RPL];
+#pragma unroll
+    for (int q = 0; q < RPL; q++) {
+        lab[q] = sh.lab[min(lane + 64 * q, n - 1)];
+        pof[q] = sh.pof[min(lane + 64 * q, n - 1)];
+    }
+    for (int c0 = wv; c0 < n; c0 += 16) {
+        float v[4][RPL];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int q = 0; q < RPL; q++) v[u][q] = A[min(lane + 64 * q, n - 1) + n * min(c0 + 4 * u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int c = c0 + 4 * u, cc = min(c, n - 1);
+            int pc = __builtin_amdgcn_readlane(pof[0], cc & 63);
+            if (RPL > 1 && cc >= 64) pc = __builtin_amdgcn_readlane(pof[RPL - 1], cc & 63);
+#pragma unroll
+            for (int q = 0; q < RPL; q++)
+                if (c < n && lane + 64 * q < n) out(lab[q], pc, v[u][q]);
+        }
+    }
+    return __builtin_amdgcn_readfirstlane(*sh.sing);
+}
+
+// LDS of the factorisation's inverse.
+template <typename T> using FactorInv = std::conditional_t<std::is_same<T, float>::value, StepShared<T>, InvShared<T>>;
+
 // The block kernels' shapes by block size: CPW = columns per wave of four (and, for the
 // MFMA products, k-steps of 4), RCH rows per lane.  A shape's unused columns cost their
 // share of the work, so the sizes in use have one that fits: 8-16 (triangles p=1-3, tets
@@ -256,7 +540,7 @@ block_inverse_kernel(int nrows, int bsz, const int *__restrict__ rowpts, const d
         for (long i = tid; i < b2; i += nth) A[i] = src[i];
         __syncthreads();
         double *dst = Dinv + row * b2;
-        const int r = wg_inverse<double, NT>(bsz, A, sh, [] {}, [&](int i, int c, double v) { dst[i + bsz * c] = v; });
+        const int r = wg_inverse<NT>(bsz, A, sh, [] {}, [&](int i, int c, double v) { dst[i + bsz * c] = v; });
         if (tid == 0 && info) info[row] = r;
         __syncthreads();
     }
@@ -758,7 +1042,7 @@ __device__ __forceinline__ void wg_load_block_coh(T *dst, const T *src, long n)
 template <typename T>
 __host__ __device__ constexpr size_t factor_lds(int bsz)
 {
-    return ((size_t)3 * bsz * bsz * sizeof(T) + 15) / 16 * 16 + InvShared<T>::bytes(bsz);
+    return ((size_t)3 * bsz * bsz * sizeof(T) + 15) / 16 * 16 + FactorInv<T>::bytes(bsz);
 }
 
 // The row of ticket t, by the whole workgroup (a barrier must lie between two calls).
@@ -778,7 +1062,7 @@ __device__ __forceinline__ void factor_row(int n, const int *__restrict__ rowpts
     const int tid = threadIdx.x, lane = tid & 63;
     const long b2 = (long)n * n;
     T *A = lds, *L = lds + b2, *Dg = lds + 2 * b2;
-    const InvShared<T> sh((char *)lds + ((size_t)3 * n * n * sizeof(T) + 15) / 16 * 16, n);
+    const FactorInv<T> sh((char *)lds + ((size_t)3 * n * n * sizeof(T) + 15) / 16 * 16, n);
     const int4 h = sch.rows[t];
     const int ri = __builtin_amdgcn_readfirstlane(h.x), d0 = __builtin_amdgcn_readfirstlane(h.y);
     const int first = __builtin_amdgcn_readfirstlane(h.z), cnt = __builtin_amdgcn_readfirstlane(h.w);
@@ -794,11 +1078,13 @@ __device__ __forceinline__ void factor_row(int n, const int *__restrict__ rowpts
     T *Mii = Mg + (long)d0 * b2;
     wg_load_block_coh(Dg, (const T *)Mii, b2);
     constexpr int NT = Tiles::NT;
-    // target block M_il -= L_ik U_kl (-L in LDS), tile column ct of it
+    // target block M_il -= L_ik U_kl (-L in LDS), tile column ct of it.  The product is summed
+    // by itself: onto the target's larger entries its rounding doubled the FP32 factors'
+    // error where the diagonal dominates.
     auto update_target = [&](T *Mil, const T *U, int ct) {
         const int lr = opaque(tl.lr), lk = opaque(tl.lk), j = ct * 16 + lr, jc = min(j, n - 1);
         T b[CPW];
-        v4 c[NT];
+        v4 c[NT], lu[NT];
 #pragma unroll
         for (int ks = 0; ks < CPW; ks++) b[ks] = coh_load(U, min(4 * ks + lk, n - 1) + n * jc);
 #pragma unroll
@@ -814,10 +1100,12 @@ __device__ __forceinline__ void factor_row(int n, const int *__restrict__ rowpts
         };
         load_a(0, a);
 #pragma unroll
+        for (int s = 0; s < NT; s++) lu[s] = (v4){(T)0, (T)0, (T)0, (T)0};
+#pragma unroll
         for (int ks = 0; ks < CPW; ks++) {
             if (ks + 1 < CPW) load_a(ks + 1, an);
 #pragma unroll
-            for (int s = 0; s < NT; s++) c[s] = Tiles::M::run(4 * ks + lk < n ? a[s] : (T)0, b[ks], c[s]);
+            for (int s = 0; s < NT; s++) lu[s] = Tiles::M::run(4 * ks + lk < n ? a[s] : (T)0, b[ks], lu[s]);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int s = 0; s < NT; s++) a[s] = an[s];
@@ -827,7 +1115,7 @@ __device__ __forceinline__ void factor_row(int n, const int *__restrict__ rowpts
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int i = s * 16 + Tiles::M::row(lk, v);
-                if (i < n && j < n) coh_store(Mil, i + n * j, (T)c[s][v]);
+                if (i < n && j < n) coh_store(Mil, i + n * j, (T)(c[s][v] + lu[s][v]));
             }
     };
     // the targets left of the current neighbour: those of the last one are updated next to
@@ -888,9 +1176,10 @@ __device__ __forceinline__ void factor_row(int n, const int *__restrict__ rowpts
         __syncthreads();
         if (act && diag) {
             v4 dg[TPW];
-            tl.each([&](int s, int v, int o) { dg[s][v] = Dg[o]; });
+#pragma unroll
+            for (int s = 0; s < TPW; s++) dg[s] = (v4){(T)0, (T)0, (T)0, (T)0};
             tl.product(L, bd, dg);
-            tl.each([&](int s, int v, int o) { Dg[o] = dg[s][v]; });
+            tl.each([&](int s, int v, int o) { Dg[o] += dg[s][v]; });
         }
         w0 = q + 1 == cnt;
         ct = tl.wv - w0;
@@ -899,7 +1188,7 @@ __device__ __forceinline__ void factor_row(int n, const int *__restrict__ rowpts
             while (pair()) {}
     }
     __syncthreads();
-    const int r = wg_inverse<T, NT>(n, Dg, sh, [&] { pair(); }, [&](int i, int c, T v) { coh_store(Mii, i + n * c, v); });
+    const int r = wg_inverse<NT>(n, Dg, sh, [&] { pair(); }, [&](int i, int c, T v) { coh_store(Mii, i + n * c, v); });
     if (tl.wv > 0)
         while (pair()) {}
     if (tid == 0) info[ri] = r;
