@@ -132,6 +132,7 @@ extern "C" int hfem_destroy(hfem_ctx *c)
         if (ev) hipEventDestroy(ev);
     for (auto &ev : c->sv.ev)
         if (ev) hipEventDestroy(ev);
+    if (c->sv.h_dots) hipHostFree(c->sv.h_dots);
     if (c->sv.apply_graph) hipGraphExecDestroy(c->sv.apply_graph);
     if (c->lin_exec) hipGraphExecDestroy(c->lin_exec);
     if (c->blas) rocblas_destroy_handle(c->blas);

@@ -115,9 +115,12 @@ hipError_t launch_bilu0_syncfree(int bsz, const int4 *lrows, const int2 *lnbr, c
 hipError_t launch_bilu0_syncfree(int bsz, const int4 *lrows, const int2 *lnbr, const int4 *urows, const int2 *unbr,
                                  int n, const float *Mg, const double *x, double *t, double *y, unsigned *sync,
                                  int nwg, int spin_limit, int *err, hipStream_t s);
-int multidot_blocks(long n);
-hipError_t launch_multidot(long n, int k, const double *V, long ldv, const double *w, double *partial, double *out,
-                           hipStream_t s);
+int gs_blocks(long n);
+hipError_t launch_gs_project(long n, int k, const double *V, long ldv, double *w, const double *pin, double *pout,
+                             double *hout, hipStream_t s);
+hipError_t launch_gs_update(long n, int k, const double *V, long ldv, double *w, const double *d, const double *pin,
+                            double *pout, double *hout, hipStream_t s);
+hipError_t launch_gs_scale(long n, const double *x, double *y, const double *pin, double *hout, hipStream_t s);
 hipError_t launch_multi_axpy(long n, int k, const double *V, long ldv, const double *coef, double sign, double *w,
                              hipStream_t s);
 hipError_t launch_axpby(long n, double a, const double *x, double b, double *y, hipStream_t s);
@@ -176,7 +179,8 @@ struct SolverState {
     double *V = nullptr;                // Krylov basis, (restart+1) columns of length N
     int vcols = 0;
     double *b = nullptr, *t = nullptr;  // preconditioned rhs, work vector
-    double *dots = nullptr;             // partial sums of the multi-dot kernel
+    double *dots = nullptr;             // partial sums of the orthogonalisation, two sets
+    double *h_dots = nullptr;           // their totals (page-locked host memory, written by the device)
     double *coef = nullptr;             // device copy of Gram-Schmidt coefficients
     double *UDGi = nullptr;             // DIRK: solution at the start of the time step
     // timings of the last calls (milliseconds; device events inside GMRES)
