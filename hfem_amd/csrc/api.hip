@@ -125,7 +125,7 @@ extern "C" int hfem_destroy(hfem_ctx *c)
                     c->r, c->partial, c->xv, c->yv, c->sv.d_u2o, c->sv.d_lsched, c->sv.d_usched,
                     c->sv.d_lnbr, c->sv.d_unbr, c->sv.d_fnbr,
                     c->sv.Mg, c->sv.Mg32, c->sv.gy, c->sv.Dinv, c->sv.Cw, c->sv.d_info, c->sv.x, c->sv.V, c->sv.b, c->sv.t, c->sv.dots,
-                    c->sv.coef, c->sv.UDGi, c->sv.sf_flags, c->sv.sf_err, c->qn_dinv, c->qn_K, c->rdmax, c->rcmax, c->rdprev, c->rcount};
+                    c->sv.coef, c->sv.UDGi, c->sv.sf_flags, c->sv.sf_err, c->qn_dinv, c->qn_K, c->rdmax, c->rcmax, c->rdprev, c->rcount, c->pack};
     for (void *p : ptrs)
         if (p) hipFree(p);
     for (auto &ev : c->ev)
@@ -775,42 +775,74 @@ extern "C" int hfem_sync(hfem_ctx *c)
     return 0;
 }
 
-// Copy the element blocks of [e0, e0+n) to the host in the reference layouts.
-// Fx (row-major, F then Ru) is transposed back to column-major F; Hx gives H
-// (first nb columns) -- before condensation -- or AH after it.
+// n elements' results of `per` doubles each to the host: pack(first element, count, dst)
+// brings them into the order the caller sees, PACK_DOUBLES at a time, and one contiguous
+// copy takes them over.  The right-hand side of 750 p=4 tets and its read-back with DinvRu
+// as a strided copy of 131 250 single doubles took 892 ms, 0.88 now; the condensation of
+// 340 tets of p = 1-4 read back with two copies per element and the transposition on the
+// host 24.7 ms, 10.5 now (of that the kernels 2.4, the rest the copies to pageable memory).
+constexpr long PACK_DOUBLES = 1L << 22;
+
+template <class F>
+static int read_packed(hfem_ctx *c, int n, long per, double *host, F pack)
+{
+    if (n <= 0) return 0;
+    long cap = std::min(n, 65535) * per;
+    if (cap > PACK_DOUBLES) cap = std::max(per, PACK_DOUBLES / per * per);
+    if (c->pack_len < cap) {
+        if (c->pack) HIPCHK(hipFree(c->pack));
+        c->pack = nullptr;
+        c->pack_len = 0;
+        // (with the device nearly full: fewer elements at a time)
+        while (hfem_dalloc(&c->pack, cap) != hipSuccess) {
+            (void)hipGetLastError();
+            c->pack = nullptr;
+            if (cap <= per) return hfem_fail(-2, "no device memory for the results of one element (%ld bytes)", 8 * per);
+            cap = std::max(per, cap / per / 2 * per);
+        }
+        c->pack_len = cap;
+    }
+    const int m = (int)std::min(65535L, c->pack_len / per);
+    for (int t = 0; t < n; t += m) {
+        const int k = std::min(m, n - t);
+        HIPCHK(pack(t, k, c->pack));
+        HIPCHK(hipMemcpyAsync(host + t * per, c->pack, sizeof(double) * k * per, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(hipStreamSynchronize(c->stream));
+    }
+    return 0;
+}
+
+// The row-major na x ldx blocks src: their first nb columns column-major, and column nb.
 static int read_rowmajor(hfem_ctx *c, const double *src, int e0, int n, double *colmajor, double *lastcol)
 {
-    const Dims &d = c->d;
-    const long na = d.na, nb = d.nb, ldx = c->ldx;
-    if (!colmajor) {
-        // the last column alone: one strided copy
-        if (lastcol && n > 0)
-            HIPCHK(hipMemcpy2D(lastcol, sizeof(double), src + (long)e0 * na * ldx + nb, sizeof(double) * ldx,
-                               sizeof(double), (size_t)n * na, hipMemcpyDeviceToHost));
-        return 0;
-    }
-    std::vector<double> tmp((size_t)n * na * ldx);
-    HIPCHK(hipMemcpy(tmp.data(), src + (long)e0 * na * ldx, sizeof(double) * tmp.size(), hipMemcpyDeviceToHost));
-    for (long t = 0; t < n; t++)
-        for (long i = 0; i < na; i++) {
-            const double *row = tmp.data() + (t * na + i) * ldx;
-            if (colmajor)
-                for (long j = 0; j < nb; j++) colmajor[t * na * nb + i + na * j] = row[j];
-            if (lastcol) lastcol[t * na + i] = row[nb];
-        }
-    return 0;
+    const long na = c->d.na, nb = c->d.nb, ldx = c->ldx;
+    const double *S = src + e0 * na * ldx;
+    int rc = 0;
+    if (colmajor)
+        rc = read_packed(c, n, na * nb, colmajor, [&](long t, int k, double *dst) {
+            return launch_pack_transposed(k, (int)na, (int)nb, (int)ldx, S + t * na * ldx, dst, c->stream);
+        });
+    if (!rc && lastcol)
+        rc = read_packed(c, n, na, lastcol, [&](long t, int k, double *dst) {
+            return launch_pack_runs(k * na, 1, ldx, S + t * na * ldx + nb, dst, c->stream);
+        });
+    return rc;
 }
 
 static int read_hx(hfem_ctx *c, int e0, int n, double *H, double *lastcol)
 {
-    const Dims &d = c->d;
-    const long nb = d.nb, es = nb * (nb + 1);
-    for (long t = 0; t < n; t++) {
-        const double *src = c->Hx + (e0 + t) * es;
-        if (H) HIPCHK(hipMemcpy(H + t * nb * nb, src, sizeof(double) * nb * nb, hipMemcpyDeviceToHost));
-        if (lastcol) HIPCHK(hipMemcpy(lastcol + t * nb, src + nb * nb, sizeof(double) * nb, hipMemcpyDeviceToHost));
-    }
-    return 0;
+    const long nb = c->d.nb, es = nb * (nb + 1);
+    const double *S = c->Hx + e0 * es;
+    int rc = 0;
+    if (H)
+        rc = read_packed(c, n, nb * nb, H, [&](long t, int k, double *dst) {
+            return launch_pack_runs(k, (int)(nb * nb), es, S + t * es, dst, c->stream);
+        });
+    if (!rc && lastcol)
+        rc = read_packed(c, n, nb, lastcol, [&](long t, int k, double *dst) {
+            return launch_pack_runs(k, (int)nb, es, S + t * es + nb * nb, dst, c->stream);
+        });
+    return rc;
 }
 
 extern "C" int hfem_read_elements(hfem_ctx *c, int e0, int n, double *Ru, double *D, double *F, double *K, double *H,

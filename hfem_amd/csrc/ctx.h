@@ -71,6 +71,8 @@ hipError_t launch_bsr_gather(int, int, int, int, int, long, const int *, const i
                              double *, hipStream_t);
 hipError_t launch_face_gather(int, int, int, int, int, long, const int *, const int *, const double *, double *,
                               const double *, double *, hipStream_t);
+hipError_t launch_pack_runs(long n, int w, long stride, const double *src, double *dst, hipStream_t s);
+hipError_t launch_pack_transposed(int n, int na, int nb, int ldx, const double *src, double *dst, hipStream_t s);
 hipError_t launch_sumsq(long, const double *, int, double *, int, hipStream_t);
 hipError_t launch_bsr_matvec(int, int, const int *, const int *, const double *, const double *, double *,
                              hipStream_t);
@@ -230,6 +232,8 @@ struct hfem_ctx {
     int prod_var[5] = {0, 0, 0, 0, 0};
     // mixed refinement: per-element maxima, previous correction, unconverged count
     unsigned long long *rdmax = nullptr, *rcmax = nullptr, *rdprev = nullptr;
+    double *pack = nullptr;      // element results on their way to the host
+    long pack_len = 0;
     int *rcount = nullptr;
     int mix_max_sweeps = 4;
     double mix_tol = 1e-11;

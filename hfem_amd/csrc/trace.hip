@@ -59,6 +59,31 @@ __global__ void face_gather_kernel(int nf, int bsz, int nch, int npf, int nb, lo
     }
 }
 
+// Element results packed for the host: runs of w doubles every `stride` (n of them).
+__global__ void __launch_bounds__(256)
+pack_runs_kernel(long n, int w, long stride, const double *__restrict__ src, double *__restrict__ dst)
+{
+    for (long i = blockIdx.x * 256L + threadIdx.x; i < n * w; i += gridDim.x * 256L) dst[i] = src[i / w * stride + i % w];
+}
+
+// Row-major na x ldx blocks, their first nb columns to column-major na x nb.  32 x 32 tiles
+// through LDS, so both sides are read and written along their rows.
+__global__ void __launch_bounds__(256)
+pack_transposed_kernel(int na, int nb, int ldx, const double *__restrict__ src, double *__restrict__ dst)
+{
+    __shared__ double tile[32][33];
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5, i0 = blockIdx.x * 32, j0 = blockIdx.y * 32;
+    const double *S = src + (long)blockIdx.z * na * ldx;
+    double *D = dst + (long)blockIdx.z * na * nb;
+#pragma unroll
+    for (int r = 0; r < 32; r += 8)
+        if (i0 + ty + r < na && j0 + tx < nb) tile[ty + r][tx] = S[(long)(i0 + ty + r) * ldx + j0 + tx];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 32; r += 8)
+        if (i0 + tx < na && j0 + ty + r < nb) D[i0 + tx + (long)na * (j0 + ty + r)] = tile[tx][ty + r];
+}
+
 // Partial sums of squares; partial[blockIdx.x] (deterministic two-stage reduction).
 __global__ void sumsq_kernel(long n, const double *__restrict__ x, int square, double *__restrict__ partial)
 {
@@ -177,6 +202,20 @@ hipError_t launch_face_gather(int nf, int bsz, int nch, int npf, int nb, long es
 {
     hipLaunchKernelGGL(face_gather_kernel, dim3(grid_for((long)nf * bsz)), dim3(256), 0, s, nf, bsz, nch, npf, nb,
                        estride, f2e, einv, V1, o1, V2, o2);
+    return hipGetLastError();
+}
+
+hipError_t launch_pack_runs(long n, int w, long stride, const double *src, double *dst, hipStream_t s)
+{
+    hipLaunchKernelGGL(pack_runs_kernel, dim3(grid_for(n * w)), dim3(256), 0, s, n, w, stride, src, dst);
+    return hipGetLastError();
+}
+
+// n blocks, at most 65535.
+hipError_t launch_pack_transposed(int n, int na, int nb, int ldx, const double *src, double *dst, hipStream_t s)
+{
+    hipLaunchKernelGGL(pack_transposed_kernel, dim3((na + 31) / 32, (nb + 31) / 32, n), dim3(256), 0, s, na, nb, ldx, src,
+                       dst);
     return hipGetLastError();
 }
 
