@@ -653,13 +653,17 @@ __device__ __forceinline__ void wave_block_matvec(int bsz, const TM *__restrict_
 //   pattern no result has (SWEEP_EMPTY) and polls the entries it needs, so a hand-over is
 //   one store and one load (about 0.45 us between any two CUs; a separate flag behind
 //   a completed store, the earlier form, put three more round trips in each link).
-// Measured per application (two sweeps), FP64 factors, before with a flag per row and
-// one wave per whole block, and now:
-//   16 464 p=3 tets (block 50, 557 levels)         3.60 ms   1.82 ms
-//   8^3 periodic p=2 hexes (block 45, 370 levels)  2.68 ms   0.75 ms
-//   4 608 p=4 triangles (block 20, 849 levels)     4.82 ms   1.43 ms
-//   512 p=2 triangles (block 12, 104 levels)       0.63 ms   0.20 ms
-// i.e. 0.85-1.0 us per link; the large mesh is bound by reading its factors (4.6 GB)
+// * Behind the last neighbour's z there is no branch, reload or readlane any more: taken
+//   branches (some 30 cycles each) and readlanes (9) were two thirds of that path.
+// Measured per application (two sweeps), FP64 factors: with a flag per row and one wave
+// per whole block; with z as the flag and a quarter of each block per wave; now:
+//   16 464 p=3 tets (block 50, 557 levels)         3.60 ms   1.81 ms   1.58 ms
+//   8^3 periodic p=2 hexes (block 45, 370 levels)  2.68 ms   0.75 ms   0.61 ms
+//   750 p=4 tets (block 75, 146 levels)            1.79 ms   0.64 ms   0.43 ms
+//   4 608 p=4 triangles (block 20, 849 levels)     4.82 ms   1.42 ms   1.28 ms
+//   512 p=2 triangles (block 12, 104 levels)       0.63 ms   0.20 ms   0.18 ms
+// i.e. 0.75-0.9 us per link, of which the hand-over 0.45 us (a store and the load that
+// sees it, between any two CUs); the large mesh is bound by reading its factors (4.6 GB)
 // next to the chain.
 struct RowSched {
     const int4 *rows;    // by ticket: row, its diagonal block, first entry in nbr, neighbours
@@ -675,27 +679,50 @@ constexpr unsigned long long SWEEP_EMPTY = 0x7ff4dead5eed0001ull;
 // set), sets *err and returns.
 __device__ __forceinline__ double wait_entry(const double *p, int spin_limit, int *err)
 {
-    unsigned long long v;
-    int spins = 0;
-    // (the ballot makes the loop's control wave-uniform)
-    while (true) {
-        v = __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (__ballot(v == SWEEP_EMPTY) == 0) break;
-        if (++spins > spin_limit ||
-            ((spins & 63) == 0 && __builtin_amdgcn_readfirstlane(
-                                      __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))) {
-            __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            break;
-        }
+    auto load = [&] {
+        return __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // (the ballot makes the loop's control wave-uniform; one exit that falls through: a
+    // taken branch costs some 30 cycles)
+    unsigned long long v = load();
+    bool waiting = __ballot(v == SWEEP_EMPTY) != 0;
+    const unsigned limit = (unsigned)spin_limit;
+    unsigned spins = 0;
+    while (__builtin_expect(waiting && spins < limit, 1)) {
         __builtin_amdgcn_s_sleep(1);
+        spins++;
+        if (__builtin_expect((spins & 63) == 0, 0) &&
+            __builtin_amdgcn_readfirstlane(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+            spins = limit;
+        v = load();
+        waiting = __ballot(v == SWEEP_EMPTY) != 0;
     }
+    if (__builtin_expect(waiting, 0)) __hip_atomic_store(err, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     return __longlong_as_double((long long)v);
+}
+
+// Lane J of every row of 16 lanes to the whole row (DPP row_newbcast).
+template <int J>
+__device__ __forceinline__ double row16_bcast(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, 0x150 + J, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + J, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+template <class F, int... J>
+__device__ __forceinline__ void for_columns(F f, std::integer_sequence<int, J...>)
+{
+    (f(std::integral_constant<int, J>()), ...);
 }
 
 // One row of a sweep, the ticket t's, by the whole workgroup.  The lane holds block
 // rows lane (+ 64 with RCH 2); wave w the columns [w cpw, (w+1) cpw) of each block,
 // cpw = ceil(bsz / 4) <= CPW.  Loads are clamped into the block and columns past the
-// wave's multiplied by zero.  Shared by the one-launch (WAIT) and level-launched
+// wave's multiplied by zero.  With one row per lane the wave's vector entries are fetched
+// by every row of 16 lanes and broadcast in it by DPP (10 cycles a column with the
+// multiplication; as readlanes 18).  Shared by the one-launch (WAIT) and level-launched
 // kernels so that both compute the same bits.
 template <bool BACKWARD, int RCH, int CPW, int NPRE, bool WAIT, typename TM>
 __device__ __forceinline__ void sweep_row(int bsz, const RowSched &sch, int t, const TM *__restrict__ Mg,
@@ -709,12 +736,18 @@ __device__ __forceinline__ void sweep_row(int bsz, const RowSched &sch, int t, c
     const int4 h = sch.rows[t];
     const int r = __builtin_amdgcn_readfirstlane(h.x), kd = __builtin_amdgcn_readfirstlane(h.y);
     const int first = __builtin_amdgcn_readfirstlane(h.z), cnt = __builtin_amdgcn_readfirstlane(h.w);
-    const int2 *nbr = sch.nbr + first;
+    // lane i: the row's neighbour i (fewer than FACTOR_MAXROW)
+    const int2 nb = sch.nbr[first + max(min(lane, cnt - 1), 0)];
+    auto block = [&](int i) { return __builtin_amdgcn_readlane(nb.x, i); };
+    auto vec = [&](int i) { return z + (long)__builtin_amdgcn_readlane(nb.y, i) * bsz; };
     int rl[RCH];
 #pragma unroll
     for (int q = 0; q < RCH; q++) rl[q] = min(lane + 64 * q, bsz - 1);
-    const int ce = min(c0 + min(lane, cpw - 1), bsz - 1);       // the vector entry this lane fetches
-    const bool cv = lane < cpw && c0 + lane < bsz;
+    // the vector entry this lane fetches
+    constexpr bool DPP = RCH == 1;
+    static_assert(!DPP || CPW <= 16, "columns per wave");
+    const int le = DPP ? lane & 15 : lane, ce = min(c0 + min(le, cpw - 1), bsz - 1);
+    const bool cv = le < cpw && c0 + le < bsz;
     auto load_share = [&](int blk, TM (&v)[CPW][RCH]) {
         const TM *B = Mg + (long)blk * b2;
 #pragma unroll
@@ -724,17 +757,22 @@ __device__ __forceinline__ void sweep_row(int bsz, const RowSched &sch, int t, c
     };
     auto add_share = [&](const TM (&v)[CPW][RCH], double ze, double (&acc)[RCH]) {
         const double zm = cv ? ze : 0.0;
-#pragma unroll
-        for (int j = 0; j < CPW; j++) {
-            const double zj = wave_bcast(zm, j);
+        for_columns([&](auto J) {
+            constexpr int j = J();
+            double zj;
+            if constexpr (DPP) zj = row16_bcast<j>(zm);
+            else zj = wave_bcast(zm, j);
 #pragma unroll
             for (int q = 0; q < RCH; q++) acc[q] += (double)v[j][q] * zj;
-        }
+        }, std::make_integer_sequence<int, CPW>());
     };
+    // the blocks of the last NPRE neighbours (base + i), the last to be waited for; the
+    // last neighbour is always the last of them, so that no branch follows its z
+    const int base = cnt - NPRE;
     TM v[NPRE][CPW][RCH];
 #pragma unroll
     for (int i = 0; i < NPRE; i++)
-        if (i < cnt) load_share(__builtin_amdgcn_readfirstlane(nbr[i].x), v[i]);
+        if (base + i >= 0) load_share(block(base + i), v[i]);
     double own[RCH], acc[RCH];
 #pragma unroll
     for (int q = 0; q < RCH; q++) {
@@ -749,15 +787,15 @@ __device__ __forceinline__ void sweep_row(int bsz, const RowSched &sch, int t, c
 #pragma unroll
         for (int q = 0; q < RCH; q++) own[q] = b[(long)r * bsz + rl[q]];
     }
-    for (int i0 = 0; i0 < cnt; i0 += NPRE) {
-#pragma unroll
-        for (int i = 0; i < NPRE; i++) {
-            if (i0 + i >= cnt) break;
-            const double *ze = z + (long)__builtin_amdgcn_readfirstlane(nbr[i0 + i].y) * bsz + ce;
-            add_share(v[i], WAIT ? wait_entry(ze, spin_limit, err) : *ze, acc);
-            if (i0 + NPRE + i < cnt) load_share(__builtin_amdgcn_readfirstlane(nbr[i0 + NPRE + i].x), v[i]);
-        }
+    auto entry_of = [&](int i) { return WAIT ? wait_entry(vec(i) + ce, spin_limit, err) : vec(i)[ce]; };
+    for (int i = 0; i < base; i++) {
+        TM u[CPW][RCH];
+        load_share(block(i), u);
+        add_share(u, entry_of(i), acc);
     }
+#pragma unroll
+    for (int i = 0; i < NPRE; i++)
+        if (base + i >= 0) add_share(v[i], entry_of(base + i), acc);
 #pragma unroll
     for (int q = 0; q < RCH; q++) red[wv][lane + 64 * q] = own[q] - acc[q];
     __syncthreads();
@@ -902,7 +940,7 @@ bilu0_scale_upper_kernel(int bsz, int n, const int *__restrict__ rowpts, const i
 // XCDs); the row's flag is stored after every wave's stores have completed.
 // FP64, before (all operands through LDS, target search by LDS scans, the inverse in
 // LDS) and now: 16 464 p=3 tets (block 50, 557 levels) 86.9 and 27.0 ms; 8^3 periodic p=2
-// hexes (block 45, 370 levels) 43.1 and 11.5 ms; 4 608 p=4 triangles (block 25, 849
+// hexes (block 45, 370 levels) 43.1 and 11.5 ms; 4 608 p=4 triangles (block 20, 849
 // levels) 37.2 and 11.9 ms.  Of a row's time in the hexes (28 us): its first neighbour's
 // flag to L 3.4 us, the targets 2.4 us, the inverse 22 us.
 
