@@ -489,17 +489,12 @@ static hipError_t run_prod(hfem_ctx *c, int which, int var, int e0, int n, const
                         (size_t)c->maxlds, c->stream);
 }
 
-// Default launch choices before any tuning: the first hand-written variant that
-// fits each product.
+// Default launch choices before any tuning: the products in their pipelined form, the
+// solves fused where that fits.
 static void default_choices(hfem_ctx *c)
 {
     const Dims &d = c->d;
-    for (int w = 0; w < 5; w++) {
-        const int M = w == 1 ? d.nb + 1 : d.na, N = w == 1 ? d.nb : d.nb + 1;
-        c->prod_var[w] = -1;
-        for (int v = 0; v < bgemm_num_variants(); v++)
-            if (bgemm_fits(prod_mode(w), v, M, N, (size_t)c->maxlds)) { c->prod_var[w] = v; break; }
-    }
+    for (int w = 0; w < 5; w++) c->prod_var[w] = bgemm_default_variant();
     for (int w = 0; w <= 2; w += 2)
         if (xsolve_fits(w == 0 ? 0 : 1, d.na, (size_t)c->maxlds)) c->prod_var[w] = kFused;
 }

@@ -334,6 +334,141 @@ static hipError_t bgemm_direct_go(const BgemmArgs &g, hipStream_t s)
     return hipGetLastError();
 }
 
+// The same without LDS, pipelined: a wave owns RT x CT tiles, its operands go from memory
+// into registers PD k-steps ahead, and C0 is fetched a tile row ahead of the results (one
+// entry at a time its latency was more than half of the Schur product).  Bound by memory:
+// X and the Schur product of na = 100, nb = 200 move 1.4 MB per element in FP64 (4.5 ms
+// for 16 464 elements at the 4.9 TB/s of a copy; their 64-cycle matrix instructions take
+// 3.3), and take 7.2 ms; the best of the others, rocBLAS's among them, 7.1 after tuning.
+// 384 elements without tuning: 424 us in the staged form, 185 now.
+// 4 x 2 tiles, two k-steps: within 3% of the best of ten shapes on tets p=2-4, hexes p=2
+// and triangles p=4, 60 to 32 768 elements (more tiles leave too few waves, more k-steps
+// too few registers).
+template <typename TM, typename TA, typename TB, int RT, int CT, int PD>
+__global__ void __launch_bounds__(256, 2)
+bgemm_pipe_kernel(BgemmArgs g)
+{
+    typedef Mf<TM> F;
+    typedef typename F::v4 v4;
+    constexpr int W = 4;
+    const int tid = threadIdx.x, lane = tid & 63, lr = lane & 15, lk = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int TR = (g.M + 15) >> 4, TC = (g.N + 15) >> 4;
+    const int nbr = (TR + RT - 1) / RT, nbc = (TC + CT - 1) / CT, nblk = nbr * nbc;
+    const int nwi = (nblk + W - 1) / W;          // workgroup items per element
+    const unsigned items = (unsigned)((g.n + 7) / 8) * 8 * nwi;
+    const int nks = (g.K + 3) >> 2;              // k-steps
+    for (unsigned it = blockIdx.x; it < items; it += gridDim.x) {
+        // (work items of one element on one XCD, as in the staged form)
+        const unsigned q = it / 8;
+        const int t = (int)(q / nwi * 8 + it % 8), wi = (int)(q % nwi);
+        const int b = wi * W + wave;
+        if (t >= g.n || b >= nblk) continue;
+        const long e = (long)g.e0 + t;
+        const int br = b / nbc, bc = b - br * nbc;
+        const TA *Ae = (const TA *)g.A + e * g.sa;
+        const TB *Be = (const TB *)g.B + e * g.sb;
+        int ia[RT], jb[CT];
+#pragma unroll
+        for (int r = 0; r < RT; r++) ia[r] = min(16 * (br * RT + r) + lr, g.M - 1);
+#pragma unroll
+        for (int c = 0; c < CT; c++) jb[c] = min(16 * (bc * CT + c) + lr, g.N - 1);
+        v4 acc[RT][CT];
+#pragma unroll
+        for (int r = 0; r < RT; r++)
+#pragma unroll
+            for (int c = 0; c < CT; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) acc[r][c][v] = (TM)0;
+        TA fa[PD][RT];
+        TB fb[PD][CT];
+        // (rows of A and B past K are clamped here and zeroed at their use)
+        auto load = [&](int ks, int buf) {
+            const int k = min(4 * ks + lk, g.K - 1), ka = k * g.lda, kb = k * g.ldb;
+#pragma unroll
+            for (int r = 0; r < RT; r++) fa[buf][r] = Ae[ka + ia[r]];
+#pragma unroll
+            for (int c = 0; c < CT; c++) fb[buf][c] = Be[kb + jb[c]];
+        };
+        auto multiply = [&](int ks, int buf) {
+            const bool kok = 4 * ks + lk < g.K;
+            TM a[RT], bb[CT];
+#pragma unroll
+            for (int r = 0; r < RT; r++) a[r] = kok ? (TM)fa[buf][r] : (TM)0;
+#pragma unroll
+            for (int c = 0; c < CT; c++) bb[c] = kok ? (TM)fb[buf][c] : (TM)0;
+#pragma unroll
+            for (int r = 0; r < RT; r++)
+#pragma unroll
+                for (int c = 0; c < CT; c++) acc[r][c] = F::mfma(a[r], bb[c], acc[r][c]);
+        };
+#pragma unroll
+        for (int u = 0; u < PD; u++) load(u, u);
+        // (no branch between the matrix instructions: k-steps past the last are of zeros)
+        for (int ks = 0; ks < nks; ks += PD) {
+#pragma unroll
+            for (int u = 0; u < PD; u++) {
+                multiply(ks + u, u);
+                load(ks + u + PD, u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        // C = beta C0 + alpha acc, C0 of one tile row ahead (one entry at a time its
+        // latency was more than half of the Schur product)
+        double *Ce = g.C + e * g.sc;
+        const double *C0e = g.C0 ? g.C0 + e * g.sc0 : nullptr;
+        unsigned long long dm = 0, cm = 0;
+        double c0[2][CT][4];
+        auto load_c0 = [&](int r, double (&x)[CT][4]) {
+#pragma unroll
+            for (int c = 0; c < CT; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++)
+                    x[c][v] = C0e[(long)min(16 * (br * RT + r) + F::row(lk, v), g.M - 1) * g.ldc0 + jb[c]];
+        };
+        if (C0e) load_c0(0, c0[0]);
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            if (C0e && r + 1 < RT) load_c0(r + 1, c0[(r + 1) & 1]);
+#pragma unroll
+            for (int c = 0; c < CT; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const int i = 16 * (br * RT + r) + F::row(lk, v), j = 16 * (bc * CT + c) + lr;
+                    const double d = g.alpha * (double)acc[r][c][v];
+                    const double y = C0e ? fma(g.beta, c0[r & 1][c][v], d) : d;
+                    if (i < g.M && j < g.N) {
+                        Ce[(long)i * g.ldc + j] = y;
+                        const unsigned long long bd = (unsigned long long)__double_as_longlong(fabs(d));
+                        const unsigned long long by = (unsigned long long)__double_as_longlong(fabs(y));
+                        dm = bd > dm ? bd : dm;
+                        cm = by > cm ? by : cm;
+                    }
+                }
+        }
+        if (g.dmax) {
+            dm = wave_max_bits(dm);
+            cm = wave_max_bits(cm);
+            if (lane == 0) {
+                atomicMax(g.dmax + t, dm);
+                atomicMax(g.cmax + t, cm);
+            }
+        }
+    }
+}
+
+template <typename TM, typename TA, typename TB>
+static hipError_t bgemm_pipe_go(const BgemmArgs &g, hipStream_t s)
+{
+    constexpr int RT = 4, CT = 2, PD = 2;
+    const int TR = (g.M + 15) / 16, TC = (g.N + 15) / 16;
+    const int nblk = ((TR + RT - 1) / RT) * ((TC + CT - 1) / CT), nwi = (nblk + 3) / 4;
+    const long items = (long)((g.n + 7) / 8) * 8 * nwi;
+    const int grid = (int)std::min<long>(items, 1 << 20);
+    hipLaunchKernelGGL((bgemm_pipe_kernel<TM, TA, TB, RT, CT, PD>), dim3(grid), dim3(256), 0, s, g);
+    return hipGetLastError();
+}
+
 // Candidate launch shapes (waves, tiles per wave, K chunk).  The tuner times the
 // ones that fit a shape; variant 0 is the default.
 struct BgemmShape {
@@ -349,7 +484,14 @@ struct DirectShape {
 static constexpr DirectShape kDirect[] = {{2, 2}, {1, 2}, {2, 4}};
 constexpr int kNumDirect = sizeof(kDirect) / sizeof(kDirect[0]);
 
-int bgemm_num_variants() { return kNumShapes + kNumDirect; }
+// After them the pipelined form.
+constexpr int kPipeVariant = kNumShapes + kNumDirect;
+
+int bgemm_num_variants() { return kPipeVariant + 1; }
+
+// The variant taken before any tuning (or without a context): the staged form took 2 to
+// 2.3 times as long.
+int bgemm_default_variant() { return kPipeVariant; }
 
 // Strips needed for variant v at M x N (0 if the variant cannot run the shape).
 static int bgemm_strips(int v, int M, int N, int esize, size_t maxlds)
@@ -392,8 +534,12 @@ static hipError_t bgemm_go(const BgemmArgs &g, size_t lds, hipStream_t s)
 // mode 0: FP64 MFMA with A, B double; mode 1: FP32 MFMA with A float, B double.
 hipError_t launch_bgemm(int mode, int variant, BgemmArgs g, size_t maxlds, hipStream_t s)
 {
-    if (variant < 0 || variant >= kNumShapes + kNumDirect) return hipErrorInvalidValue;
+    if (variant < 0 || variant > kPipeVariant) return hipErrorInvalidValue;
     if (g.n <= 0) return hipSuccess;
+    if (variant == kPipeVariant) {
+        g.nstrip = 1;
+        return mode == 0 ? bgemm_pipe_go<double, double, double>(g, s) : bgemm_pipe_go<float, float, double>(g, s);
+    }
     if (variant >= kNumShapes) {
         g.nstrip = 1;
 #define HFEM_BD(V)                                                                                                 \
@@ -425,7 +571,7 @@ hipError_t launch_bgemm(int mode, int variant, BgemmArgs g, size_t maxlds, hipSt
 // Whether variant v can run an M x N product (strips fit registers and LDS).
 bool bgemm_fits(int mode, int variant, int M, int N, size_t maxlds)
 {
-    if (variant >= kNumShapes && variant < kNumShapes + kNumDirect) return M > 0 && N > 0;
+    if (variant >= kNumShapes && variant <= kPipeVariant) return M > 0 && N > 0;
     if (variant < 0 || variant >= kNumShapes) return false;
     return bgemm_strips(variant, M, N, mode == 0 ? 8 : 4, maxlds) > 0;
 }

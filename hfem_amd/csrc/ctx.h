@@ -54,6 +54,7 @@ struct BgemmArgs {
     unsigned long long *dmax, *cmax;  // optional per-element maxima (index e - e0)
 };
 int bgemm_num_variants();
+int bgemm_default_variant();
 // xsolve.hip: fused per-element solve X = inv(D)[F Ru] (mode 0 FP64, mode 1 mixed)
 bool xsolve_fits(int mode, int na, size_t maxlds);
 hipError_t launch_xsolve(int mode, int na, int N, int ldx, int e0, int n, const double *D, const void *inv,

@@ -59,15 +59,7 @@ extern "C" int hfem_condense_noalloc(int na, int nb, int ldx, int n, const doubl
     int rc = scratch_for_device(dev, &inv, &maxlds);
     if (rc) return rc;
     hipStream_t s = (hipStream_t)stream;
-    // the first hand-written variant that fits each product (the context's
-    // default choice)
-    auto pick = [&](int M, int N) {
-        for (int v = 0; v < bgemm_num_variants(); v++)
-            if (bgemm_fits(0, v, M, N, (size_t)maxlds)) return v;
-        return -1;
-    };
-    const int v0 = pick(na, nb + 1), v1 = pick(nb + 1, nb);
-    if (v0 < 0 || v1 < 0) return hfem_fail(-1, "hfem_condense_noalloc: no product kernel fits na=%d nb=%d", na, nb);
+    const int var = bgemm_default_variant();   // the context's default choice
     HIPCHK(launch_dinv(na, 0, n, D, inv, info, s, 0));
     const long sx = (long)na * ldx, sd = (long)na * na, sk = (long)nb * na, sh = (long)nb * (nb + 1);
     BgemmArgs g{};
@@ -79,7 +71,7 @@ extern "C" int hfem_condense_noalloc(int na, int nb, int ldx, int n, const doubl
     g.B = Fx; g.sb = sx; g.ldb = ldx;
     g.alpha = 1.0; g.beta = 0.0;
     g.C = X; g.sc = sx; g.ldc = ldx;
-    HIPCHK(launch_bgemm(0, v0, g, (size_t)maxlds, s));
+    HIPCHK(launch_bgemm(0, var, g, (size_t)maxlds, s));
     // [AH FH] = [H Rh] - K X, as AH^T = H^T - X^T K^T
     g = BgemmArgs{};
     g.e0 = 0;
@@ -90,6 +82,6 @@ extern "C" int hfem_condense_noalloc(int na, int nb, int ldx, int n, const doubl
     g.alpha = -1.0; g.beta = 1.0;
     g.C0 = Hx; g.sc0 = sh; g.ldc0 = nb;
     g.C = Hx; g.sc = sh; g.ldc = nb;
-    HIPCHK(launch_bgemm(0, v1, g, (size_t)maxlds, s));
+    HIPCHK(launch_bgemm(0, var, g, (size_t)maxlds, s));
     return 0;
 }
