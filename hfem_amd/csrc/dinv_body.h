@@ -506,6 +506,11 @@ __device__ __forceinline__ void dinv_body(int na, int e0, int n, const double *_
 #pragma unroll
                     for (int ks = 0; ks < 4; ks++)
                         a[s] = G::mfma(pan[(r * 16 + lr) * PS + ks * 4 + lk], Z[(ks * 4 + lk) * NN + q * 16 + lr], a[s]);
+                    // (the tile may be read on the far side of a taken branch, where the compiler
+                    // was seen to leave too few wait states behind the last of these: 8 of 18,
+                    // 3 of 10 in FP32)
+                    if constexpr (sizeof(T) == 4) asm volatile("s_nop 7\n\ts_nop 3" : "+v"(a[s]));
+                    else asm volatile("s_nop 15\n\ts_nop 3" : "+v"(a[s]));
                 }
             }
             __syncthreads();

@@ -4,10 +4,10 @@
 blocks are diagonally dominant (condition below 10), so an entry's error is a few na
 roundings of its sums: 1e-12 relative to the largest entry.
 """
-import ctypes
-
 import numpy as np
 import pytest
+
+from test_zz_no_alloc import DeviceBuffers
 
 pytestmark = pytest.mark.gpu
 
@@ -16,7 +16,6 @@ pytestmark = pytest.mark.gpu
                                      (32, 64, 1), (33, 65, 17), (60, 60, 8), (64, 127, 3), (65, 128, 2), (100, 200, 5),
                                      (135, 270, 3), (176, 300, 2)])
 def test_condense_shapes(na, nb, n):
-    import torch
     from hfem_amd.lib import load
     rng = np.random.default_rng(na * 1000 + nb)
     ldx = nb + 1 + na % 3
@@ -24,19 +23,16 @@ def test_condense_shapes(na, nb, n):
     Fx = rng.standard_normal((n, na, ldx))
     K = rng.standard_normal((n, na, nb))
     H = rng.standard_normal((n, nb + 1, nb))
-    t = {k: torch.from_numpy(v.copy()).cuda() for k, v in dict(D=D, Fx=Fx, K=K, H=H).items()}
-    X = torch.full((n, na, ldx), 7.0, dtype=torch.float64, device="cuda")
-    info = torch.zeros(n, dtype=torch.int32, device="cuda")
+    X0 = np.full((n, na, ldx), 7.0)
+    buf = DeviceBuffers()
+    p = {k: buf.upload(v) for k, v in dict(D=D, Fx=Fx, K=K, H=H, X=X0, info=np.zeros(n, np.int32)).items()}
     print(f"na {na} nb {nb} n {n}", flush=True)
-    rc = load().hfem_condense_noalloc(na, nb, ldx, n, *[ctypes.c_void_p(t[k].data_ptr()) for k in ("D", "Fx", "K", "H")],
-                                      ctypes.c_void_p(X.data_ptr()), ctypes.c_void_p(info.data_ptr()),
-                                      torch.cuda.current_stream().cuda_stream)
-    assert rc == 0
-    torch.cuda.synchronize()
+    assert load().hfem_condense_noalloc(na, nb, ldx, n, p["D"], p["Fx"], p["K"], p["H"], p["X"], p["info"], None) == 0
+    got, gotH, info = buf.download(p["X"], X0), buf.download(p["H"], H), buf.download(p["info"], np.zeros(n, np.int32))
+    buf.free()
     want = np.linalg.solve(D.transpose(0, 2, 1), Fx[:, :, :nb + 1])
-    got = X.cpu().numpy()
-    assert not info.cpu().numpy().any()
+    assert not info.any()
     assert np.abs(got[:, :, :nb + 1] - want).max() <= 1e-12 * np.abs(want).max()
     assert (got[:, :, nb + 1:] == 7.0).all()
     wantH = H - np.einsum("eai,eaj->eij", want, K)
-    assert np.abs(t["H"].cpu().numpy() - wantH).max() <= 1e-12 * na * np.abs(wantH).max()
+    assert np.abs(gotH - wantH).max() <= 1e-12 * na * np.abs(wantH).max()
