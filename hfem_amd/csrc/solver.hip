@@ -546,40 +546,6 @@ block_inverse_kernel(int nrows, int bsz, const int *__restrict__ rowpts, const d
     }
 }
 
-// MDF block weights C(n) = ||inv(H_ii) H_n||_F for every block n of row i
-// (kernel/computeMDFordering.m:14-20).  One workgroup per row.
-__global__ void __launch_bounds__(SV_THREADS)
-mdf_weight_kernel(int nrows, int bsz, const int *__restrict__ rowpts, const double *__restrict__ Hg,
-                  const double *__restrict__ Dinv, double *__restrict__ Cw)
-{
-    extern __shared__ double lds[];
-    const int tid = threadIdx.x, nth = blockDim.x;
-    const long b2 = (long)bsz * bsz;
-    double *A = lds, *B = lds + b2, *red = lds + 2 * b2;
-    for (int row = blockIdx.x; row < nrows; row += gridDim.x) {
-        for (long i = tid; i < b2; i += nth) A[i] = Dinv[row * b2 + i];
-        for (int n = rowpts[row]; n < rowpts[row + 1]; n++) {
-            for (long i = tid; i < b2; i += nth) B[i] = Hg[(long)n * b2 + i];
-            __syncthreads();
-            double s2 = 0.0;
-            for (long idx = tid; idx < b2; idx += nth) {
-                const int i = idx % bsz, j = idx / bsz;
-                double s = 0.0;
-                for (int k = 0; k < bsz; k++) s += A[i + bsz * k] * B[k + bsz * j];
-                s2 += s * s;
-            }
-            red[tid] = s2;
-            __syncthreads();
-            for (int st = nth / 2; st > 0; st >>= 1) {
-                if (tid < st) red[tid] += red[tid + st];
-                __syncthreads();
-            }
-            if (tid == 0) Cw[n] = sqrt(red[0]);
-            __syncthreads();
-        }
-    }
-}
-
 // Broadcast lane `src` (wave-uniform) of a double to the whole wave.
 __device__ __forceinline__ double wave_bcast(double v, int src)
 {
@@ -1003,7 +969,8 @@ struct BlockTiles {
         lk = lane >> 4;
         wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     }
-    __device__ bool active() const { return NT == 1 ? wv == 0 : NT == 3 ? wv < 3 : true; }
+    static constexpr __device__ int waves() { return NT == 1 ? 1 : NT == 3 ? 3 : 4; }
+    __device__ bool active() const { return wv < waves(); }
     __device__ bool has(int s) const { return s < 6 || wv == 0; }
     __device__ int rt(int s) const { return NT == 2 ? wv >> 1 : s < 5 ? s : s == 5 ? wv : 4; }
     __device__ int cb(int s) const { return s < 5 ? 0 : 1; }
@@ -1061,6 +1028,62 @@ struct BlockTiles {
                 }
     }
 };
+
+// MDF block weights C(n) = ||inv(H_ii) H_n||_F for every block n of row i
+// (kernel/computeMDFordering.m:14-20).  One workgroup per row, inv(H_ii) in LDS, the other
+// blocks straight from memory into the B operands, the next block's while the current is
+// multiplied; only sums of squares leave the registers.  Floor: reading the matrix, 1 ms for
+// 34 104 rows of 50 x 50 blocks (4.8 GB); 8.9 ms as a dot product per thread out of LDS,
+// 2.4 ms now.
+constexpr int MDF_BATCH = 32;   // blocks between two barriers
+
+template <int CPW>
+__global__ void __launch_bounds__(SV_THREADS, CPW <= 16 ? 2 : 1)
+mdf_weight_kernel(int nrows, int bsz, const int *__restrict__ rowpts, const double *__restrict__ Hg,
+                  const double *__restrict__ Dinv, double *__restrict__ Cw)
+{
+    extern __shared__ double lds[];
+    __shared__ double red[MDF_BATCH][SV_THREADS / 64];
+    typedef BlockTiles<double, CPW> Tiles;
+    const Tiles tl(bsz);
+    const int tid = threadIdx.x, lane = tid & 63;
+    const long b2 = (long)bsz * bsz;
+    const bool act = tl.active();
+    for (int row = blockIdx.x; row < nrows; row += gridDim.x) {
+        const int n0 = __builtin_amdgcn_readfirstlane(rowpts[row]), n1 = __builtin_amdgcn_readfirstlane(rowpts[row + 1]);
+        for (long i = tid; i < b2; i += SV_THREADS) lds[i] = Dinv[row * b2 + i];
+        __syncthreads();
+        for (int m0 = n0; m0 < n1; m0 += MDF_BATCH) {
+            const int m1 = min(m0 + MDF_BATCH, n1);
+            if (act) {
+                double b[Tiles::NCB][CPW], bn[Tiles::NCB][CPW];
+                tl.load_b(Hg + (long)m0 * b2, b);
+                for (int n = m0; n < m1; n++) {
+                    tl.load_b(Hg + (long)min(n + 1, m1 - 1) * b2, bn);
+                    typename Tiles::v4 acc[Tiles::TPW];
+#pragma unroll
+                    for (int s = 0; s < Tiles::TPW; s++) acc[s] = (typename Tiles::v4){0.0, 0.0, 0.0, 0.0};
+                    tl.product(lds, b, acc);
+                    double s2 = 0.0;
+                    tl.each([&](int s, int v, int) { s2 += acc[s][v] * acc[s][v]; });
+                    for (int d = 32; d > 0; d >>= 1) s2 += __shfl_xor(s2, d);
+                    if (lane == 0) red[n - m0][tl.wv] = s2;
+#pragma unroll
+                    for (int c = 0; c < Tiles::NCB; c++)
+#pragma unroll
+                        for (int ks = 0; ks < CPW; ks++) b[c][ks] = bn[c][ks];
+                }
+            }
+            __syncthreads();
+            if (m0 + tid < m1) {
+                double s2 = 0.0;
+                for (int w = 0; w < SV_THREADS / 64; w++) s2 += Tiles::waves() > w ? red[tid][w] : 0.0;
+                Cw[m0 + tid] = sqrt(s2);
+            }
+            __syncthreads();
+        }
+    }
+}
 
 // dst[i] = src[i] for i < n by the workgroup, eight loads in flight per thread.
 template <typename T>
@@ -1598,17 +1621,6 @@ hipError_t launch_block_inverse(int nrows, int bsz, const int *rowpts, const dou
     return hipGetLastError();
 }
 
-hipError_t launch_mdf_weights(int nrows, int bsz, const int *rowpts, const double *Hg, const double *Dinv,
-                              double *Cw, hipStream_t s)
-{
-    const size_t lds = sizeof(double) * (2 * bsz * bsz + SV_THREADS);
-    hipError_t e = set_lds((const void *)mdf_weight_kernel, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(mdf_weight_kernel, dim3(std::min(nrows, 8192)), dim3(SV_THREADS), lds, s, nrows, bsz, rowpts,
-                       Hg, Dinv, Cw);
-    return hipGetLastError();
-}
-
 // (block sizes above 80 have no factorisation shape: bilu0_factor_lds)
 template <class F>
 static hipError_t factor_shape(int bsz, F launch)
@@ -1616,6 +1628,15 @@ static hipError_t factor_shape(int bsz, F launch)
     if (bsz > 80) return hipErrorInvalidValue;
     return block_shape(bsz, [&](auto R, auto C) {
         if constexpr (C() <= 20) launch(R, C);
+    });
+}
+
+hipError_t launch_mdf_weights(int nrows, int bsz, const int *rowpts, const double *Hg, const double *Dinv,
+                              double *Cw, hipStream_t s)
+{
+    return factor_shape(bsz, [&](auto, auto C) {
+        hipLaunchKernelGGL(mdf_weight_kernel<C()>, dim3(std::min(nrows, 8192)), dim3(SV_THREADS),
+                           sizeof(double) * bsz * bsz, s, nrows, bsz, rowpts, Hg, Dinv, Cw);
     });
 }
 
