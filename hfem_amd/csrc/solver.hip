@@ -839,48 +839,6 @@ sweep_reset_kernel(unsigned *sync, long n, double *t, double *y)
     }
 }
 
-// The factorisation's last step for the sweeps: every upper block of row r becomes
-// U~_rl = inv(U_rr) U_rl (inv(U_rr) is the row's diagonal block), in place, after
-// the whole factorisation (the other rows' eliminations read the unscaled U_rl).
-// One workgroup per row: inv(U_rr) in LDS (FP64), the upper blocks a few columns
-// at a time, each thread one entry of inv(U_rr) times a staged column.
-template <typename TM>
-__global__ void __launch_bounds__(SV_THREADS)
-bilu0_scale_upper_kernel(int bsz, int n, const int *__restrict__ rowpts, const int *__restrict__ colind,
-                         const int *__restrict__ u2o, TM *__restrict__ Mg)
-{
-    extern __shared__ double su[];
-    const long b2 = (long)bsz * bsz;
-    const int tid = threadIdx.x, cpp = max(1, SV_THREADS / bsz);
-    double *Dl = su, *Cl = su + b2;
-    for (int r = blockIdx.x; r < n; r += gridDim.x) {
-        // (row bounds and the upper test through readfirstlane: loop control with
-        // barriers inside must be uniform)
-        const int k0 = __builtin_amdgcn_readfirstlane(rowpts[r]);
-        const int len = __builtin_amdgcn_readfirstlane(rowpts[r + 1]) - k0;
-        const int o = __builtin_amdgcn_readfirstlane(u2o[r]);
-        const TM *Ui = Mg + (long)k0 * b2;
-        for (long i = tid; i < b2; i += SV_THREADS) Dl[i] = (double)Ui[i];
-        __syncthreads();
-        for (int q = 1; q < len; q++) {
-            if (__builtin_amdgcn_readfirstlane(u2o[colind[k0 + q]]) <= o) continue;
-            TM *B = Mg + (long)(k0 + q) * b2;
-            for (int c0 = 0; c0 < bsz; c0 += cpp) {
-                const int nc = min(cpp, bsz - c0);
-                for (int i = tid; i < nc * bsz; i += SV_THREADS) Cl[i] = (double)B[(long)c0 * bsz + i];
-                __syncthreads();
-                if (tid < nc * bsz) {
-                    const int c = tid / bsz, i = tid - c * bsz;
-                    double acc = 0.0;
-                    for (int k = 0; k < bsz; k++) acc += Dl[i + (long)bsz * k] * Cl[c * bsz + k];
-                    B[(long)(c0 + c) * bsz + i] = (TM)acc;
-                }
-                __syncthreads();
-            }
-        }
-    }
-}
-
 // ---- BILU0 factorisation (kernel/computeBILU0.m) ----
 //
 // In the row-oriented form: row i takes, for each neighbour k numbered before it,
@@ -976,13 +934,14 @@ struct BlockTiles {
     __device__ int cb(int s) const { return s < 5 ? 0 : 1; }
     __device__ int ct(int b) const { return b ? 4 : NT == 2 ? (wv & 1) : wv; }
     // B operands: every k-step of the wave's tile columns of a block in global memory
-    __device__ __forceinline__ void load_b(const T *B, T (&b)[NCB][CPW]) const
+    template <typename S>
+    __device__ __forceinline__ void load_b(const S *B, T (&b)[NCB][CPW]) const
     {
 #pragma unroll
         for (int c = 0; c < NCB; c++) {
             const int col = min(ct(c) * 16 + opaque(lr), n - 1), k = opaque(lk);
 #pragma unroll
-            for (int ks = 0; ks < CPW; ks++) b[c][ks] = coh_load(B, min(4 * ks + k, n - 1) + n * col);
+            for (int ks = 0; ks < CPW; ks++) b[c][ks] = (T)coh_load(B, min(4 * ks + k, n - 1) + n * col);
         }
     }
     // acc += A b with A in LDS (rows past n are computed and not stored; k past n is
@@ -1082,6 +1041,73 @@ mdf_weight_kernel(int nrows, int bsz, const int *__restrict__ rowpts, const doub
             }
             __syncthreads();
         }
+    }
+}
+
+// The factorisation's last step for the sweeps: every upper block of row r becomes
+// U~_rl = inv(U_rr) U_rl (inv(U_rr) is the row's diagonal block), in place, after
+// the whole factorisation (the other rows' eliminations read the unscaled U_rl).
+// One workgroup per row, as mdf_weight_kernel: inv(U_rr) in LDS (FP64 for either type of
+// factors), the upper blocks straight from memory into the B operands, the next one's
+// while the current is multiplied.  Floor: the upper blocks read and written and the
+// diagonal ones read, 1 ms for 34 104 rows of 50 x 50 blocks (4.7 GB).  As a dot product
+// per thread out of LDS and now: those 2.55 and 1.76 ms, 1 536 rows of 45 x 45 243 and
+// 94 us, 375 of them in single precision 180 and 40, 7 008 of 20 x 20 in single precision
+// 32 and 41 (a wave's one tile per block is too little to cover its latency; 0.01% of
+// that solve, so there is one form).
+template <int CPW, typename TM>
+__global__ void __launch_bounds__(SV_THREADS, CPW <= 16 ? 2 : 1)
+bilu0_scale_upper_kernel(int bsz, int n, const int *__restrict__ rowpts, const int *__restrict__ colind,
+                         const int *__restrict__ u2o, TM *__restrict__ Mg)
+{
+    extern __shared__ double lds[];
+    typedef BlockTiles<double, CPW> Tiles;
+    const Tiles tl(bsz);
+    const int lane = threadIdx.x & 63;
+    const long b2 = (long)bsz * bsz;
+    const bool act = tl.active();
+    for (int r = blockIdx.x; r < n; r += gridDim.x) {
+        // (loop control with barriers inside must be uniform)
+        const int k0 = __builtin_amdgcn_readfirstlane(rowpts[r]);
+        const int len = __builtin_amdgcn_readfirstlane(rowpts[r + 1]) - k0;
+        const int o = __builtin_amdgcn_readfirstlane(u2o[r]);
+        const TM *Ui = Mg + (long)k0 * b2;
+        for (long i = threadIdx.x; i < b2; i += SV_THREADS) lds[i] = (double)Ui[i];
+        __syncthreads();
+        for (int q0 = 1; q0 < len; q0 += 64) {
+            // lane l: whether block q0 + l is an upper one
+            const int q = min(q0 + lane, len - 1);
+            unsigned long long todo = __ballot(q0 + lane < len && u2o[colind[k0 + q]] > o);
+            if (!todo) continue;
+            int m = __ffsll((long long)todo) - 1;
+            double b[Tiles::NCB][CPW], bn[Tiles::NCB][CPW];
+            if (act) tl.load_b((const TM *)Mg + (long)(k0 + q0 + m) * b2, b);
+            while (true) {
+                TM *B = Mg + (long)(k0 + q0 + m) * b2;
+                todo &= todo - 1;
+                if (todo) m = __ffsll((long long)todo) - 1;
+                typename Tiles::v4 acc[Tiles::TPW];
+                if (act) {
+                    tl.load_b((const TM *)Mg + (long)(k0 + q0 + m) * b2, bn);
+#pragma unroll
+                    for (int s = 0; s < Tiles::TPW; s++) acc[s] = (typename Tiles::v4){0.0, 0.0, 0.0, 0.0};
+                    tl.product(lds, b, acc);
+                    // (18 wait states behind an FP64 matrix instruction: the compiler leaves
+                    // too few where its result is stored on the far side of a taken branch)
+#pragma unroll
+                    for (int s = 0; s < Tiles::TPW; s++) asm volatile("s_nop 15\n\ts_nop 3" : "+v"(acc[s]));
+                }
+                // (two waves read a tile column: both have their operands before either stores)
+                if constexpr (Tiles::NT == 2 || Tiles::NT == 5) __syncthreads();
+                if (act) tl.each([&](int s, int v, int i) { *entry(B, i) = (TM)acc[s][v]; });
+                if (!todo) break;
+#pragma unroll
+                for (int c = 0; c < Tiles::NCB; c++)
+#pragma unroll
+                    for (int ks = 0; ks < CPW; ks++) b[c][ks] = bn[c][ks];
+            }
+        }
+        __syncthreads();
     }
 }
 
@@ -1702,12 +1728,10 @@ static hipError_t scale_upper(int bsz, int n, const int *rowpts, const int *coli
                               hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    const size_t lds = sizeof(double) * ((size_t)bsz * bsz + (size_t)std::max(1, SV_THREADS / bsz) * bsz);
-    hipError_t e = set_lds((const void *)bilu0_scale_upper_kernel<TM>, lds);
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(bilu0_scale_upper_kernel<TM>, dim3(std::min(n, 16384)), dim3(SV_THREADS), lds, s, bsz, n,
-                       rowpts, colind, u2o, Mg);
-    return hipGetLastError();
+    return factor_shape(bsz, [&](auto, auto C) {
+        hipLaunchKernelGGL((bilu0_scale_upper_kernel<C(), TM>), dim3(std::min(n, 8192)), dim3(SV_THREADS),
+                           sizeof(double) * bsz * bsz, s, bsz, n, rowpts, colind, u2o, Mg);
+    });
 }
 hipError_t launch_bilu0_scale_upper(int bsz, int n, const int *rowpts, const int *colind, const int *u2o,
                                     double *Mg, hipStream_t s)
