@@ -15,6 +15,17 @@ constexpr int ASM_LDS_MAX = 160 * 1024;   // LDS per workgroup on gfx950
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
+// The wait behind a wave's last matrix instruction (an FP64 one's result takes 18 wait
+// states), a its result: the compiler, which counts them up to the result's use, leaves 15
+// or 16 where it is stored, and 10 of 11 where its register is written again, on the far
+// side of a taken branch.  At the end of a k-loop, so it costs nothing that shows (16 464
+// p=3 tets 14.26 and 14.36 ms on two cards).
+__device__ __forceinline__ void mfma_settle(f64x4 &a)
+{
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n\ts_nop 3" : "+v"(a));
+}
+
 // LDS layout of the assembly kernel in doubles (the int tables follow).  Master
 // tables are transposed so that the thread-varying index is fastest:
 // svt[n + npv*(g + ngv*dd)], svg[i + npv*(g + ngv*dd)] (as shapvg),
@@ -597,6 +608,7 @@ assemble_body(const Dims &d, const Master &m, const Phys &ph, const double *__re
                                 // ahead of the products (they would not fit in registers)
                                 __builtin_amdgcn_sched_barrier(0);
                             }
+                    mfma_settle(acc[NT - 1]);
 #pragma unroll
                     for (int t = 0; t < NT; t++)
 #pragma unroll
@@ -741,6 +753,7 @@ assemble_body(const Dims &d, const Master &m, const Phys &ph, const double *__re
                         const double qv = Qm[k + CS * (ngv + pp)];
                         acc = __builtin_amdgcn_mfma_f64_16x16x4f64(k0 + lk < npv ? qv : 0.0, bsrc[k], acc, 0, 0, 0);
                     }
+                    mfma_settle(acc);
 #pragma unroll
                     for (int v = 0; v < 4; v++) {
                         const int gr = rg * 16 + lk + 4 * v;
@@ -810,6 +823,7 @@ assemble_body(const Dims &d, const Master &m, const Phys &ph, const double *__re
                             for (int t = 0; t < NT; t++) acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(aq[x][t], bq, acc[t], 0, 0, 0);
                         }
                     }
+                    mfma_settle(acc[NT - 1]);
                     // result: lane holds C(row = l/16 + 4v, col = l%16) of each tile
                     const int colc = ct * 16 + lr;
                     if (colc < ncol) {
