@@ -39,17 +39,29 @@ static int ensure_vectors(hfem_ctx *c, int restart)
     if (!s.d_info) HIPCHK(hfem_dalloc(&s.d_info, (size_t)c->hd.nf));
     for (auto &e : s.ev)
         if (!e) HIPCHK(hipEventCreate(&e));
-    if (restart + 1 > s.vcols) {
-        if (s.V) HIPCHK(hipFree(s.V));
-        if (s.dots) HIPCHK(hipFree(s.dots));
-        if (s.coef) HIPCHK(hipFree(s.coef));
-        if (s.h_dots) HIPCHK(hipHostFree(s.h_dots));
-        s.V = s.dots = s.coef = s.h_dots = nullptr;
-        s.vcols = restart + 1;
-        HIPCHK(hfem_dalloc(&s.V, (size_t)N * s.vcols));
-        HIPCHK(hfem_dalloc(&s.dots, 2 * (size_t)gs_blocks(N) * s.vcols));
-        HIPCHK(hipHostMalloc((void **)&s.h_dots, sizeof(double) * (2 * (size_t)s.vcols + 1), hipHostMallocDefault));
-        HIPCHK(hfem_dalloc(&s.coef, (size_t)s.vcols + 1));
+    const size_t cols = (size_t)restart + 1;
+    if (cols > (size_t)s.vcols) {
+        // (no columns until all four are there, so that a call after a failed one tries again)
+        auto release = [&] {
+            s.vcols = 0;
+            for (double **p : {&s.V, &s.dots, &s.coef}) {
+                if (*p) (void)hipFree(*p);
+                *p = nullptr;
+            }
+            if (s.h_dots) (void)hipHostFree(s.h_dots);
+            s.h_dots = nullptr;
+        };
+        release();
+        hipError_t e = hfem_dalloc(&s.V, N * cols);
+        if (e == hipSuccess) e = hfem_dalloc(&s.dots, 2 * (size_t)gs_blocks(N) * cols);
+        if (e == hipSuccess) e = hipHostMalloc((void **)&s.h_dots, sizeof(double) * (2 * cols + 1), hipHostMallocDefault);
+        if (e == hipSuccess) e = hfem_dalloc(&s.coef, cols + 1);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            release();
+            return hfem_fail(-2, "no memory for a Krylov basis of %zu vectors of %ld entries: %s", cols, N, hipGetErrorString(e));
+        }
+        s.vcols = (int)cols;
     }
     return 0;
 }
