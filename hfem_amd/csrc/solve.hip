@@ -526,9 +526,10 @@ static int bilu0_sweeps(hfem_ctx *c, const double *x, double *y)
     return 0;
 }
 
-// How the BILU0 sweeps run: mode 1 (default) one persistent launch per sweep whose
-// workgroups wait on per-row ready flags, each wait bounded by spin_limit polls (0:
-// the default 2^20), a wait that gives up making the next hfem_gmres /
+// How BILU0 runs: mode 1 (default) one persistent launch for the factorisation, whose
+// workgroups wait on per-row ready flags, and one per sweep, whose workgroups wait on the
+// vector entries themselves; each wait is bounded by spin_limit polls (0: the default
+// 2^20), one that gives up making the next hfem_precond_factor / hfem_gmres /
 // hfem_precond_apply fail; mode 0 one launch per level.  Same bits either way.  No
 // counterpart in the reference.
 extern "C" int hfem_set_bilu0_sweep(hfem_ctx *c, int mode, int spin_limit)
@@ -542,9 +543,10 @@ extern "C" int hfem_set_bilu0_sweep(hfem_ctx *c, int mode, int spin_limit)
     return 0;
 }
 
-// Whether the level-by-level BILU0 application replays a captured graph (1, default) or
-// launches its levels one by one (0).  (The persistent sweeps are three launches, cheaper
-// than a graph's launch and the copy out of its fixed output: 4.4 us on 132 300 unknowns.)  No counterpart in the reference.
+// Whether the BILU0 application replays a captured graph of its launches (1) or launches
+// them one by one (0, default: the persistent sweeps are three launches, 4.4 us cheaper on
+// 132 300 unknowns than a graph's launch and the copy out of its fixed output).  No
+// counterpart in the reference.
 extern "C" int hfem_set_apply_graph(hfem_ctx *c, int use)
 {
     if (!c) return hfem_fail(-1, "hfem_set_apply_graph: null context");
@@ -567,8 +569,8 @@ static int precond_apply_dev(hfem_ctx *c, const double *x, double *y)
     } else if (s.prec == 0) {
         const long bytes = sizeof(double) * N;
         if (s.sweep_mode == 1) RC(ensure_syncfree(c));
-        if (s.use_graph && s.sweep_mode == 0) {
-            // the level launches of both sweeps as one graph from c->yv into s.gy
+        if (s.use_graph) {
+            // the launches of both sweeps as one graph from c->yv into s.gy
             // (captured after each factorisation; no memset nodes in it)
             if (s.graph_dirty || !s.apply_graph) {
                 if (s.apply_graph) HIPCHK(hipGraphExecDestroy(s.apply_graph));

@@ -343,13 +343,13 @@ class HDGContext:
         _check(load().hfem_set_linearization_graph(self.h, int(bool(use))))
 
     def set_apply_graph(self, use=True):
-        """Replay the BILU0 application as a captured HIP graph, or launch its
-        levels one by one (default)."""
+        """Replay the BILU0 application, in either mode of set_bilu0_sweep, as a
+        captured HIP graph, or launch its sweeps one by one (default)."""
         _check(load().hfem_set_apply_graph(self.h, int(use)))
 
     def set_bilu0_sweep(self, mode, spin_limit=0):
-        """BILU0 sweeps as one persistent launch per sweep with bounded per-row
-        waits (mode 1, default) or level by level (mode 0)."""
+        """BILU0 factorisation and sweeps as one persistent launch each with bounded
+        waits for the rows they read (mode 1, default) or level by level (mode 0)."""
         _check(load().hfem_set_bilu0_sweep(self.h, int(mode), int(spin_limit)))
 
     def apply_preconditioner(self, x):

@@ -233,18 +233,21 @@ int hfem_precond_factor(hfem_ctx *ctx, int kind);
  * MFMA, sweeps reading FP32 factors with FP64 arithmetic), 1 in double (default).
  * Takes effect at the next hfem_precond_factor. */
 int hfem_set_precond_precision(hfem_ctx *ctx, int prec_precision);
-/* No counterpart in the reference: 1 replays the BILU0 application (the
- * level-by-level launches of both sweeps) as a HIP graph captured once per
- * factorisation; 0 (default) launches the levels one by one.  Measured equal on
- * MI355X: a sweep is bound by the latency of its chain of dependent levels, not
+/* No counterpart in the reference: 1 replays the BILU0 application (the launches
+ * of both sweeps, in either mode of hfem_set_bilu0_sweep) as a HIP graph captured
+ * once per factorisation; 0 (default) launches them one by one.  Same results bit
+ * for bit.  On MI355X 0 is the faster by some 4 us an application in mode 1 (three
+ * launches); a sweep is bound by the latency of its chain of dependent rows, not
  * by launch overhead. */
 int hfem_set_apply_graph(hfem_ctx *ctx, int use);
 /* No counterpart in the reference (kernel/applyBILU0.m runs its sweeps row by
- * row): mode 1 (default) runs each BILU0 sweep as one persistent launch whose
- * workgroups take the rows in level order and wait on per-row ready flags, each
- * wait bounded by spin_limit polls (0: 2^20); mode 0 launches the sweeps level by
- * level.  Same results bit for bit.  A wait that gives up makes the next
- * hfem_gmres / hfem_precond_apply return an error. */
+ * row): mode 1 (default) runs the BILU0 factorisation and each sweep as one
+ * persistent launch whose workgroups take the rows in level order and wait for the
+ * rows they read (the factorisation on a flag per row, a sweep on the entries of
+ * its vector), each wait bounded by spin_limit polls (0: 2^20); mode 0 launches
+ * them level by level.  Same results bit for bit.  A wait that gives up makes that
+ * hfem_precond_factor, or the next hfem_gmres / hfem_precond_apply, return an
+ * error. */
 int hfem_set_bilu0_sweep(hfem_ctx *ctx, int mode, int spin_limit);
 /* y = M^{-1} x with host vectors of length nf*bsz (kernel/applyBILU0.m:1-52). */
 int hfem_precond_apply(hfem_ctx *ctx, const double *x, double *y);
