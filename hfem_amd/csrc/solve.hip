@@ -78,7 +78,10 @@ static int require_system(hfem_ctx *c, const char *who)
 // Level schedules of the two BILU0 sweeps for the current ordering: a row's
 // forward level is one more than the largest forward level of its neighbours
 // numbered before it, its backward level likewise over the neighbours numbered
-// after it.  Rows of one level never depend on each other.
+// after it.  Rows of one level never depend on each other.  Neighbours in the forward
+// levels are the rows with a block on either side of the diagonal (a mesh's graph has
+// both, a caller's need not): two rows with one differ in level by the order of their
+// numbers, so a row that has both as neighbours may take them by level (ensure_schedule).
 static int build_levels(hfem_ctx *c)
 {
     SolverState &s = c->sv;
@@ -88,11 +91,13 @@ static int build_levels(hfem_ctx *c)
     int nl = 0, nu = 0;
     for (int j = 0; j < n; j++) {
         const int r = s.o2u[j];
-        int l = 0;
+        int l = lv[r];
         for (int k = rp[r] + 1; k < rp[r + 1]; k++)
             if (s.u2o[ci[k]] < j) l = std::max(l, lv[ci[k]] + 1);
         lv[r] = l;
         nl = std::max(nl, l + 1);
+        for (int k = rp[r] + 1; k < rp[r + 1]; k++)
+            if (s.u2o[ci[k]] > j) lv[ci[k]] = std::max(lv[ci[k]], l + 1);
     }
     for (int j = n - 1; j >= 0; j--) {
         const int r = s.o2u[j];

@@ -1,0 +1,80 @@
+"""Trace graphs a caller may pass beyond the mesh's own (GPU): rows in any order, further
+blocks on one side of the diagonal only.
+
+BILU0 takes a row's neighbours in the order of their numbers (kernel/computeBILU0.m):
+against that elimination in numpy to 1e-10 relative, the tolerance of the other
+preconditioner tests.
+"""
+import numpy as np
+import pytest
+
+from hfem_amd.problem import make_problem
+
+pytestmark = pytest.mark.gpu
+
+
+def widened(mesh, rng):
+    """The mesh's graph with 3 further columns a row, its rows shuffled."""
+    start, cols = [0], []
+    for i in range(mesh.nf):
+        row = list(mesh.ent2ent[mesh.ent2entStart[i] + 1:mesh.ent2entStart[i + 1]])
+        row += list(rng.permutation(np.setdiff1d(np.arange(mesh.nf), row + [i]))[:3])
+        cols += [i] + list(rng.permutation(row))
+        start.append(len(cols))
+    mesh.ent2entStart, mesh.ent2ent = np.array(start, dtype=np.int64), np.array(cols, dtype=np.int64)
+
+
+def first_in_row(rp, ci, row, col):
+    return next((m for m in range(rp[row] + 1, rp[row + 1]) if ci[m] == col), -1)
+
+
+def bilu0(rp, ci, o2u, u2o, B):
+    for r in o2u:
+        lower = [k for k in range(rp[r] + 1, rp[r + 1]) if u2o[ci[k]] < u2o[r]]
+        for k in sorted(lower, key=lambda k: u2o[ci[k]]):
+            B[k] = B[k] @ B[rp[ci[k]]]
+            for l in range(rp[r], rp[r + 1]):
+                m = first_in_row(rp, ci, ci[k], ci[l])
+                if m >= 0 and (l == rp[r] or u2o[ci[l]] > u2o[ci[k]]):
+                    B[l] -= B[k] @ B[m]
+        B[rp[r]] = np.linalg.inv(B[rp[r]])
+
+
+def bilu0_solve(rp, ci, o2u, u2o, B, x):
+    v = x.reshape(len(o2u), -1).copy()
+    for r in o2u:
+        for k in range(rp[r] + 1, rp[r + 1]):
+            if u2o[ci[k]] < u2o[r]:
+                v[r] -= B[k] @ v[ci[k]]
+    for r in o2u[::-1]:
+        for k in range(rp[r] + 1, rp[r + 1]):
+            if u2o[ci[k]] > u2o[r]:
+                v[r] -= B[k] @ v[ci[k]]
+        v[r] = B[rp[r]] @ v[r]
+    return v.reshape(-1)
+
+
+@pytest.mark.parametrize("kind,nc,p,seed", [("tri", 3, 2, 0), ("tri", 4, 1, 1), ("tet", 1, 2, 2)])
+def test_bilu0(kind, nc, p, seed):
+    from hfem_amd.lib import HDGContext
+    rng = np.random.default_rng(seed)
+    prob = make_problem(kind, nc, p, seed=3, angle=0.3, elevation=0.2)
+    widened(prob.mesh, rng)
+    rp, ci, n = prob.mesh.ent2entStart, prob.mesh.ent2ent, prob.mesh.nf
+    ctx = HDGContext(prob)
+    ctx.assemble_linear_system()
+    bsz = prob.UH.size // n
+    B = ctx.read_system()[0].reshape(-1, bsz, bsz).transpose(0, 2, 1).copy()
+    x = rng.standard_normal(n * bsz)
+    o2u = rng.permutation(n)
+    u2o = np.argsort(o2u)
+    bilu0(rp, ci, o2u, u2o, B)
+    want = bilu0_solve(rp, ci, o2u, u2o, B, x)
+    for mode in (0, 1):
+        ctx.set_bilu0_sweep(mode)
+        ctx.set_ordering(o2u)
+        ctx.compute_preconditioner(0)
+        err = np.linalg.norm(ctx.apply_preconditioner(x) - want) / np.linalg.norm(want)
+        print(f"{kind}{nc} p{p} mode {mode}: {n} rows, relative error {err:.1e}", flush=True)
+        assert err < 1e-10
+    ctx.close()
