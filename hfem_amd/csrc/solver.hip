@@ -1236,9 +1236,9 @@ __device__ __forceinline__ void factor_row(int n, const int *__restrict__ rowpts
             __syncthreads();
         }
         wg_load_block_coh(A, (const T *)Mik, b2);
-        // lane l: position of the row's column l in row k, and the mask of targets
+        // lane l: (first) position of the row's column l in row k, and the mask of targets
         km = -1;
-        for (int m = 1; m < klen; m++) km = __builtin_amdgcn_readlane(ncol, m) == rcol ? m : km;
+        for (int m = klen - 1; m > 0; m--) km = __builtin_amdgcn_readlane(ncol, m) == rcol ? m : km;
         todo = __ballot(lane < len && km > 0 && (lane == 0 || rord > ork));
         __syncthreads();
         if (WAIT) wait_ready(flags + rk, epoch, spin_limit, err);

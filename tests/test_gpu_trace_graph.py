@@ -1,8 +1,8 @@
 """Trace graphs a caller may pass beyond the mesh's own (GPU): rows in any order, further
-blocks on one side of the diagonal only.
+blocks on one side of the diagonal only, a column listed twice.
 
-BILU0 takes a row's neighbours in the order of their numbers (kernel/computeBILU0.m):
-against that elimination in numpy to 1e-10 relative, the tolerance of the other
+BILU0 takes a row's neighbours in the order of their numbers and the first block of a
+column (kernel/computeBILU0.m): against that elimination in numpy to 1e-10 relative, the tolerance of the other
 preconditioner tests.
 """
 import numpy as np
@@ -13,13 +13,16 @@ from hfem_amd.problem import make_problem
 pytestmark = pytest.mark.gpu
 
 
-def widened(mesh, rng):
-    """The mesh's graph with 3 further columns a row, its rows shuffled."""
+def widened(mesh, rng, extra=3, twice=False):
+    """The mesh's graph with `extra` further columns a row, its rows shuffled; with `twice`
+    a column of every other row again at its end."""
     start, cols = [0], []
     for i in range(mesh.nf):
         row = list(mesh.ent2ent[mesh.ent2entStart[i] + 1:mesh.ent2entStart[i + 1]])
-        row += list(rng.permutation(np.setdiff1d(np.arange(mesh.nf), row + [i]))[:3])
+        row += list(rng.permutation(np.setdiff1d(np.arange(mesh.nf), row + [i]))[:extra])
         cols += [i] + list(rng.permutation(row))
+        if twice and i % 2:
+            cols.append(cols[start[-1] + 1])
         start.append(len(cols))
     mesh.ent2entStart, mesh.ent2ent = np.array(start, dtype=np.int64), np.array(cols, dtype=np.int64)
 
@@ -54,12 +57,13 @@ def bilu0_solve(rp, ci, o2u, u2o, B, x):
     return v.reshape(-1)
 
 
+@pytest.mark.parametrize("extra,twice", [(3, False), (0, True), (3, True)], ids=["one_sided", "twice", "both"])
 @pytest.mark.parametrize("kind,nc,p,seed", [("tri", 3, 2, 0), ("tri", 4, 1, 1), ("tet", 1, 2, 2)])
-def test_bilu0(kind, nc, p, seed):
+def test_bilu0(kind, nc, p, seed, extra, twice):
     from hfem_amd.lib import HDGContext
     rng = np.random.default_rng(seed)
     prob = make_problem(kind, nc, p, seed=3, angle=0.3, elevation=0.2)
-    widened(prob.mesh, rng)
+    widened(prob.mesh, rng, extra, twice)
     rp, ci, n = prob.mesh.ent2entStart, prob.mesh.ent2ent, prob.mesh.nf
     ctx = HDGContext(prob)
     ctx.assemble_linear_system()
