@@ -2,8 +2,10 @@
 blocks on one side of the diagonal only, a column listed twice.
 
 BILU0 takes a row's neighbours in the order of their numbers and the first block of a
-column (kernel/computeBILU0.m): against that elimination in numpy to 1e-10 relative, the tolerance of the other
-preconditioner tests.
+column (kernel/computeBILU0.m), MDF weights count pairs of unnumbered neighbours
+(kernel/computeMDFordering.m), a block the graph does not have being zero: against those in
+numpy, to 1e-10 relative, the tolerance of the other preconditioner tests, and the same
+permutation.
 """
 import numpy as np
 import pytest
@@ -57,6 +59,33 @@ def bilu0_solve(rp, ci, o2u, u2o, B, x):
     return v.reshape(-1)
 
 
+def mdf(rp, ci, H):
+    n = len(rp) - 1
+    C = np.array([np.linalg.norm(np.linalg.solve(H[rp[i]], H[k])) for i in range(n) for k in range(rp[i], rp[i + 1])])
+    numbered = np.zeros(n, bool)
+
+    def weight(k):
+        s = 0.0
+        nbr = [m for m in range(rp[k] + 1, rp[k + 1]) if not numbered[ci[m]]]
+        for i in nbr:
+            back = first_in_row(rp, ci, ci[i], k)
+            near = set(ci[rp[ci[i]]:rp[ci[i] + 1]])
+            for j in nbr:
+                if j != i and ci[j] not in near and back >= 0:
+                    s += (C[back] * C[j]) ** 2
+        return np.sqrt(s)
+
+    w, order = np.array([weight(k) for k in range(n)]), []
+    for _ in range(n):
+        p = int(np.argmin(np.where(numbered, np.inf, w)))
+        order.append(p)
+        numbered[p] = True
+        for k in ci[rp[p] + 1:rp[p + 1]]:
+            if not numbered[k]:
+                w[k] = weight(k)
+    return np.array(order)
+
+
 @pytest.mark.parametrize("extra,twice", [(3, False), (0, True), (3, True)], ids=["one_sided", "twice", "both"])
 @pytest.mark.parametrize("kind,nc,p,seed", [("tri", 3, 2, 0), ("tri", 4, 1, 1), ("tet", 1, 2, 2)])
 def test_bilu0(kind, nc, p, seed, extra, twice):
@@ -81,4 +110,21 @@ def test_bilu0(kind, nc, p, seed, extra, twice):
         err = np.linalg.norm(ctx.apply_preconditioner(x) - want) / np.linalg.norm(want)
         print(f"{kind}{nc} p{p} mode {mode}: {n} rows, relative error {err:.1e}", flush=True)
         assert err < 1e-10
+    ctx.close()
+
+
+@pytest.mark.parametrize("extra,twice", [(0, False), (3, False), (0, True), (3, True)],
+                         ids=["shuffled", "one_sided", "twice", "both"])
+@pytest.mark.parametrize("kind,nc,p,seed", [("tri", 3, 2, 0), ("tri", 4, 1, 1), ("tet", 1, 2, 2)])
+def test_mdf_ordering(kind, nc, p, seed, extra, twice):
+    from hfem_amd.lib import HDGContext
+    prob = make_problem(kind, nc, p, seed=3, angle=0.3, elevation=0.2)
+    widened(prob.mesh, np.random.default_rng(seed), extra, twice)
+    ctx = HDGContext(prob)
+    ctx.assemble_linear_system()
+    bsz = prob.UH.size // prob.mesh.nf
+    H = ctx.read_system()[0].reshape(-1, bsz, bsz).transpose(0, 2, 1)
+    ctx.compute_ordering(1)
+    print(f"{kind}{nc} p{p}: {prob.mesh.nf} rows", flush=True)
+    assert np.array_equal(ctx.get_ordering()[0], mdf(prob.mesh.ent2entStart, prob.mesh.ent2ent, H))
     ctx.close()
