@@ -195,6 +195,17 @@ extern "C" int hfem_set_mesh(hfem_ctx *c, const double *dgnodes, const int *elco
     const Dims &d = c->d;
     const int ne = c->hd.ne, nf = c->hd.nf;
     if (rowstart[0] != 0 || rowstart[nf] != nblocks) return hfem_fail(-1, "hfem_set_mesh: rowstart inconsistent with nblocks");
+    // (before anything is indexed by them or replaced)
+    for (int i = 0; i < nf; i++)
+        if (rowstart[i + 1] <= rowstart[i])
+            return hfem_fail(-1, "hfem_set_mesh: row %d of the trace graph must start with its diagonal block", i);
+    for (int i = 0; i < nf; i++) {
+        if (cols[rowstart[i]] != i)
+            return hfem_fail(-1, "hfem_set_mesh: row %d of the trace graph must start with its diagonal block", i);
+        for (int k = rowstart[i]; k < rowstart[i + 1]; k++)
+            if (cols[k] < 0 || cols[k] >= nf)
+                return hfem_fail(-1, "hfem_set_mesh: row %d of the trace graph lists column %d of %d", i, cols[k], nf);
+    }
     // the trace-system buffers are sized by the first mesh's block count
     if (c->has_mesh && nblocks != c->nblocks)
         return hfem_fail(-1, "hfem_set_mesh: the trace graph has %d blocks, this context's has %d (create a new "
@@ -253,9 +264,6 @@ extern "C" int hfem_set_mesh(hfem_ctx *c, const double *dgnodes, const int *elco
     c->sv.order_method = -1;
     c->sv.prec = -2;
     c->sv.graph_dirty = true;
-    for (int i = 0; i < nf; i++)
-        if (rowstart[i + 1] <= rowstart[i] || cols[rowstart[i]] != i)
-            return hfem_fail(-1, "hfem_set_mesh: row %d of the trace graph must start with its diagonal block", i);
     const long bsz = (long)d.nch * d.npf;
     if (!c->Hg) HIPCHK(dalloc(&c->Hg, (size_t)nblocks * bsz * bsz));
     if (!c->Rg) HIPCHK(dalloc(&c->Rg, (size_t)nf * bsz));

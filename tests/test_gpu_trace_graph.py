@@ -128,3 +128,27 @@ def test_mdf_ordering(kind, nc, p, seed, extra, twice):
     print(f"{kind}{nc} p{p}: {prob.mesh.nf} rows", flush=True)
     assert np.array_equal(ctx.get_ordering()[0], mdf(prob.mesh.ent2entStart, prob.mesh.ent2ent, H))
     ctx.close()
+
+
+@pytest.mark.parametrize("column", [-1, 33, 2 ** 31 - 1], ids=["negative", "rows", "largest"])
+def test_column_out_of_range_is_refused(column):
+    """A further block with such a column is refused, and the mesh set before stays in use."""
+    from hfem_amd.lib import HDGContext, HfemError, _d, _f64, _i, _i32, load
+    prob = make_problem("tri", 3, 2, seed=3, angle=0.3, elevation=0.2)
+    mesh = prob.mesh
+    assert mesh.nf == 33
+    mesh.ent2entStart[-1] += 1
+    mesh.ent2ent = np.append(mesh.ent2ent, 0)
+    ctx = HDGContext(prob)
+    ctx.assemble_linear_system()
+    ctx.compute_preconditioner(0)
+    x = np.random.default_rng(0).standard_normal(prob.UH.size)
+    want = ctx.apply_preconditioner(x)
+    mesh.ent2ent[-1] = column
+    with pytest.raises(HfemError, match="column"):
+        HDGContext(prob)
+    rc = load().hfem_set_mesh(ctx.h, _d(_f64(prob.dgnodes_ref())), _i(_i32(mesh.elcon)), _i(_i32(mesh.bf)),
+                              _i(_i32(mesh.t2f)), _i(_i32(mesh.ent2entStart)), _i(_i32(mesh.ent2ent)), len(mesh.ent2ent))
+    assert rc != 0
+    assert np.array_equal(ctx.apply_preconditioner(x), want)
+    ctx.close()
