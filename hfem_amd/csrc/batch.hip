@@ -160,7 +160,7 @@ __global__ void __launch_bounds__(512) batch_dinv_kernel(BatchArgs A)
         switch (A.code[b]) {
 #define X(NT, v, W, GR)                                                                                          \
         case NT * 4 + v:                                                                                         \
-            dinv_body<double, double, NT, W, GR>(E.d.na, 0, E.n, E.D, E.dinv, E.info, (char *)bi_lds, src);      \
+            dinv_body<double, double, NT, W, GR, true>(E.d.na, 0, E.n, E.D, E.dinv, E.info, (char *)bi_lds, src); \
             break;
             HFEM_BATCH_INV(X)
 #undef X

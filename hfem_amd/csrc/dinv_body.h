@@ -320,7 +320,14 @@ __host__ __device__ constexpr int dinv_group_lds()
 // of a workgroup run in lockstep through the same barriers: a group whose
 // element lies beyond n repeats group 0's element and stores nothing.  lds:
 // GR group regions of dinv_group_lds<T, NT>() bytes.
-template <typename T, typename TO, int NT, int W, int GR, class Src>
+// EACH: whether a wait stands behind every tile's matrix instructions, or one behind the
+// last tile's.  The compiler counts a result's wait states (18 in FP64, 10 in FP32), but
+// was seen to leave 8 and 3 where the use lies on the far side of a taken branch: behind
+// the loop, which the one wait covers, and, in the FP32 shapes of up to five tiles a side
+// and the ragged batch's kernel, in copies of the tile at its end.
+// (tests/test_mfma_waits.py counts them in the built library.)  16 464 blocks of 100 x 100:
+// 3.35 ms with a wait behind every tile, 3.28 with one; in FP32 2.42 and 2.38.
+template <typename T, typename TO, int NT, int W, int GR, bool EACH = sizeof(T) == 4 && NT <= 5, class Src>
 __device__ __forceinline__ void dinv_body(int na, int e0, int n, const double *__restrict__ D, TO *__restrict__ Dinv,
                                           int *__restrict__ info, char *lds, Src &src)
 {
@@ -506,12 +513,15 @@ __device__ __forceinline__ void dinv_body(int na, int e0, int n, const double *_
 #pragma unroll
                     for (int ks = 0; ks < 4; ks++)
                         a[s] = G::mfma(pan[(r * 16 + lr) * PS + ks * 4 + lk], Z[(ks * 4 + lk) * NN + q * 16 + lr], a[s]);
-                    // (the tile may be read on the far side of a taken branch, where the compiler
-                    // was seen to leave too few wait states behind the last of these: 8 of 18,
-                    // 3 of 10 in FP32)
-                    if constexpr (sizeof(T) == 4) asm volatile("s_nop 7\n\ts_nop 3" : "+v"(a[s]));
-                    else asm volatile("s_nop 15\n\ts_nop 3" : "+v"(a[s]));
+                    if constexpr (EACH) {
+                        if constexpr (sizeof(T) == 4) asm volatile("s_nop 7\n\ts_nop 3" : "+v"(a[s]));
+                        else asm volatile("s_nop 15\n\ts_nop 3" : "+v"(a[s]));
+                    }
                 }
+            }
+            if constexpr (!EACH) {
+                if constexpr (sizeof(T) == 4) asm volatile("s_nop 7\n\ts_nop 3");
+                else asm volatile("s_nop 15\n\ts_nop 3");
             }
             __syncthreads();
         }
