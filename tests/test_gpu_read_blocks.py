@@ -40,3 +40,39 @@ def test_ranges_and_single_outputs(kind, nc, p):
         # (backward error of an explicit inverse: cond(D) * 2^-53, cond(D) < 1e6 here)
         assert np.abs(D @ got - want).max() <= 1e-9 * np.abs(want).max()
     ctx.close()
+
+
+def test_reads_of_several_chunks():
+    """162 p=4 tets: 8.5 M doubles of DinvF and 14.6 M of AH, more than the staging buffer
+    takes at once.  Elements at the chunks' edges read one by one give the same bits, also
+    with the buffer sized by a smaller read before, and D DinvF = F either side of an edge."""
+    from hfem_amd.lib import HDGContext, load
+    prob = make_problem("tet", 3, 4, seed=8)
+    na, nb, ne = prob.dims["na"], prob.dims["nb"], prob.ne
+    cap = 1 << 22
+    ctx = HDGContext(prob)
+    ctx.assemble_element_matrix_vector()
+    fh = np.zeros((2, nb))
+    ctx.schur_element_matrix_vector()
+    ctx.sync()
+    assert load().hfem_read_condensed(ctx.h, 0, 2, None, None, None, fh.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
+                                      None) == 0
+    whole = ctx.read_condensed()
+    assert np.array_equal(fh, whole["FH"][:2])
+    edges = {0, ne - 1}
+    for per in (na * nb, nb * nb):
+        m = cap // per
+        assert 1 < m < ne and ne % m
+        edges |= {e for e in range(m - 1, ne, m)} | {e for e in range(m, ne, m)}
+    for e in sorted(edges):
+        print(f"element {e} of {ne}", flush=True)
+        one = ctx.read_condensed(e, 1)
+        for k in whole:
+            assert np.array_equal(one[k][0], whole[k][e]), k
+    ctx.assemble_element_matrix_vector()
+    for e in (cap // (na * nb) - 1, cap // (na * nb)):
+        el = ctx.read_elements(e, 1)
+        D, F = el["D"][0].reshape(na, na).T, el["F"][0].reshape(nb, na).T
+        # (backward error of an explicit inverse: cond(D) * 2^-53, cond(D) < 1e6 here)
+        assert np.abs(D @ whole["DinvF"][e].reshape(nb, na).T - F).max() <= 1e-9 * np.abs(F).max()
+    ctx.close()
