@@ -145,7 +145,7 @@ static int ensure_schedule(hfem_ctx *c)
         for (int t = 0; t < n; t++) {
             const int r = rows[t], first = (int)nbr.size();
             for (int k = rp[r] + 1; k < rp[r + 1]; k++)
-                if ((s.u2o[ci[k]] < s.u2o[r]) == lower) nbr.push_back(make_int2(k, ci[k]));
+                if (lower ? s.u2o[ci[k]] < s.u2o[r] : s.u2o[ci[k]] > s.u2o[r]) nbr.push_back(make_int2(k, ci[k]));
             std::sort(nbr.begin() + first, nbr.end(), [&](const int2 &a, const int2 &b) {
                 return lev[a.y] != lev[b.y] ? lev[a.y] < lev[b.y] : s.u2o[a.y] < s.u2o[b.y];
             });

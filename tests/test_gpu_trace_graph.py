@@ -1,5 +1,5 @@
 """Trace graphs a caller may pass beyond the mesh's own (GPU): rows in any order, further
-blocks on one side of the diagonal only, a column listed twice.
+blocks on one side of the diagonal only, a column or the diagonal listed twice.
 
 BILU0 takes a row's neighbours in the order of their numbers and the first block of a
 column (kernel/computeBILU0.m), MDF weights count pairs of unnumbered neighbours
@@ -15,16 +15,16 @@ from hfem_amd.problem import make_problem
 pytestmark = pytest.mark.gpu
 
 
-def widened(mesh, rng, extra=3, twice=False):
-    """The mesh's graph with `extra` further columns a row, its rows shuffled; with `twice`
-    a column of every other row again at its end."""
+def widened(mesh, rng, extra, twice):
+    """The mesh's graph with `extra` further columns a row, its rows shuffled, and again at
+    the end of every other row its entry `twice` (0: the diagonal, None: none)."""
     start, cols = [0], []
     for i in range(mesh.nf):
         row = list(mesh.ent2ent[mesh.ent2entStart[i] + 1:mesh.ent2entStart[i + 1]])
         row += list(rng.permutation(np.setdiff1d(np.arange(mesh.nf), row + [i]))[:extra])
         cols += [i] + list(rng.permutation(row))
-        if twice and i % 2:
-            cols.append(cols[start[-1] + 1])
+        if twice is not None and i % 2:
+            cols.append(cols[start[-1] + twice])
         start.append(len(cols))
     mesh.ent2entStart, mesh.ent2ent = np.array(start, dtype=np.int64), np.array(cols, dtype=np.int64)
 
@@ -86,7 +86,8 @@ def mdf(rp, ci, H):
     return np.array(order)
 
 
-@pytest.mark.parametrize("extra,twice", [(3, False), (0, True), (3, True)], ids=["one_sided", "twice", "both"])
+@pytest.mark.parametrize("extra,twice", [(3, None), (0, 1), (3, 1), (0, 0)],
+                         ids=["one_sided", "twice", "both", "diagonal"])
 @pytest.mark.parametrize("kind,nc,p,seed", [("tri", 3, 2, 0), ("tri", 4, 1, 1), ("tet", 1, 2, 2)])
 def test_bilu0(kind, nc, p, seed, extra, twice):
     from hfem_amd.lib import HDGContext
@@ -113,8 +114,8 @@ def test_bilu0(kind, nc, p, seed, extra, twice):
     ctx.close()
 
 
-@pytest.mark.parametrize("extra,twice", [(0, False), (3, False), (0, True), (3, True)],
-                         ids=["shuffled", "one_sided", "twice", "both"])
+@pytest.mark.parametrize("extra,twice", [(0, None), (3, None), (0, 1), (3, 1), (0, 0)],
+                         ids=["shuffled", "one_sided", "twice", "both", "diagonal"])
 @pytest.mark.parametrize("kind,nc,p,seed", [("tri", 3, 2, 0), ("tri", 4, 1, 1), ("tet", 1, 2, 2)])
 def test_mdf_ordering(kind, nc, p, seed, extra, twice):
     from hfem_amd.lib import HDGContext
