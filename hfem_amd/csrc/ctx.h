@@ -157,6 +157,7 @@ struct SolverState {
     std::vector<int> lrows, urows;      // rows of each level, concatenated
     std::vector<int> llev, ulev;        // level of each row
     bool sched_valid = false;           // the device copies below are the current ordering's
+    bool fnbr_valid = false;            // d_fnbr (of single-precision factors) too
     // the sweeps' rows in level order with their neighbours (RowSched, solver.hip)
     int4 *d_lsched = nullptr, *d_usched = nullptr;
     int2 *d_lnbr = nullptr, *d_unbr = nullptr, *d_fnbr = nullptr;

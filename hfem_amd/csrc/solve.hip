@@ -132,7 +132,8 @@ static int build_levels(hfem_ctx *c)
 static int ensure_schedule(hfem_ctx *c)
 {
     SolverState &s = c->sv;
-    if (s.sched_valid) return 0;
+    const bool fp32 = s.prec_fp32 != 0;
+    if (s.sched_valid && (s.fnbr_valid || !fp32)) return 0;
     const int n = c->hd.nf;
     const std::vector<int> &rp = s.rowpts, &ci = s.colind;
     // the sweeps' rows in level order, each with the neighbours it reads by increasing
@@ -152,32 +153,41 @@ static int ensure_schedule(hfem_ctx *c)
             sched[t] = make_int4(r, rp[r], first, (int)nbr.size() - first);
         }
     };
-    std::vector<int4> lsched, usched;
-    std::vector<int2> lnbr, unbr;
-    schedule(s.lrows, s.llev, true, lsched, lnbr);
-    schedule(s.urows, s.ulev, false, usched, unbr);
+    std::vector<int4> sched;
+    std::vector<int2> nbr;
+    // (each list of neighbours holds at most every off-diagonal block)
+    auto upload = [&](int4 **d_sched, int2 **d_nbr) -> int {
+        if (d_sched) {
+            if (!*d_sched) HIPCHK(hfem_dalloc(d_sched, (size_t)n));
+            HIPCHK(hipMemcpy(*d_sched, sched.data(), sizeof(int4) * n, hipMemcpyHostToDevice));
+        }
+        if (!*d_nbr) HIPCHK(hfem_dalloc(d_nbr, ci.size()));
+        HIPCHK(hipMemcpy(*d_nbr, nbr.data(), sizeof(int2) * nbr.size(), hipMemcpyHostToDevice));
+        return 0;
+    };
+    if (!s.sched_valid) {
+        schedule(s.urows, s.ulev, false, sched, nbr);
+        RC(upload(&s.d_usched, &s.d_unbr));
+    }
+    schedule(s.lrows, s.llev, true, sched, nbr);
+    if (!s.sched_valid) {
+        RC(upload(&s.d_lsched, &s.d_lnbr));
+        if (!s.d_u2o) HIPCHK(hfem_dalloc(&s.d_u2o, (size_t)n));
+        HIPCHK(hipMemcpy(s.d_u2o, s.u2o.data(), sizeof(int) * n, hipMemcpyHostToDevice));
+        s.sched_valid = true;
+        s.fnbr_valid = false;
+    }
     // The single-precision factorisation's by increasing number: the order of a target's
     // updates, and with it the roundings, which can grow along the rows (solver.hip), then
     // do not depend on the levels.  In double precision, where they are far below the
     // solver's tolerances, by level: 27 ms against 29 on 16 464 p=3 tets.
-    std::vector<int2> fnbr = lnbr;
-    for (const int4 &h : lsched)
-        std::sort(fnbr.begin() + h.z, fnbr.begin() + h.z + h.w,
-                  [&](const int2 &a, const int2 &b) { return s.u2o[a.y] < s.u2o[b.y]; });
-    if (!s.d_lsched) HIPCHK(hfem_dalloc(&s.d_lsched, (size_t)n));
-    if (!s.d_usched) HIPCHK(hfem_dalloc(&s.d_usched, (size_t)n));
-    // (each holds at most every off-diagonal block)
-    if (!s.d_lnbr) HIPCHK(hfem_dalloc(&s.d_lnbr, ci.size()));
-    if (!s.d_unbr) HIPCHK(hfem_dalloc(&s.d_unbr, ci.size()));
-    if (!s.d_fnbr) HIPCHK(hfem_dalloc(&s.d_fnbr, ci.size()));
-    if (!s.d_u2o) HIPCHK(hfem_dalloc(&s.d_u2o, (size_t)n));
-    HIPCHK(hipMemcpy(s.d_lsched, lsched.data(), sizeof(int4) * n, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(s.d_usched, usched.data(), sizeof(int4) * n, hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(s.d_lnbr, lnbr.data(), sizeof(int2) * lnbr.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(s.d_unbr, unbr.data(), sizeof(int2) * unbr.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(s.d_fnbr, fnbr.data(), sizeof(int2) * fnbr.size(), hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(s.d_u2o, s.u2o.data(), sizeof(int) * n, hipMemcpyHostToDevice));
-    s.sched_valid = true;
+    if (fp32) {
+        for (const int4 &h : sched)
+            std::sort(nbr.begin() + h.z, nbr.begin() + h.z + h.w,
+                      [&](const int2 &a, const int2 &b) { return s.u2o[a.y] < s.u2o[b.y]; });
+        RC(upload(nullptr, &s.d_fnbr));
+        s.fnbr_valid = true;
+    }
     return 0;
 }
 

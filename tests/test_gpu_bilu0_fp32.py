@@ -37,3 +37,29 @@ def test_error_against_double(kind, nc, p):
     assert np.array_equal(got[0], got[1])
     assert err < 300 * 2.0 ** -24
     ctx.close()
+
+
+def test_precision_after_the_other():
+    """Factors of either precision after those of the other, in the same and in a new ordering:
+    the bits of a context that has only ever had the one."""
+    from hfem_amd.lib import HDGContext
+    prob = make_problem("tet", 2, 3, seed=3, angle=0.3, elevation=0.2)
+    x = np.random.default_rng(2).standard_normal(prob.UH.size)
+
+    def context():
+        c = HDGContext(prob)
+        c.assemble_linear_system()
+        return c
+
+    ctx, before = context(), None
+    for order, prec in [(1, 1), (1, 0), (0, 0), (1, 0), (0, 1), (0, 0), (1, 1)]:
+        fresh = context()
+        for c in (ctx, fresh):
+            if c is fresh or order != before:
+                c.compute_ordering(order)
+            c.compute_preconditioner(0, prec)
+        before = order
+        print(f"ordering {order} precision {prec}", flush=True)
+        assert np.array_equal(ctx.apply_preconditioner(x), fresh.apply_preconditioner(x))
+        fresh.close()
+    ctx.close()
