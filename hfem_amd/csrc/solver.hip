@@ -502,22 +502,23 @@ template <typename T> using FactorInv = std::conditional_t<std::is_same<T, float
 
 // The block kernels' shapes by block size: CPW = columns per wave of four (and, for the
 // MFMA products, k-steps of 4), RCH rows per lane.  A shape's unused columns cost their
-// share of the work, so the sizes in use have one that fits: 8-16 (triangles p=1-3, tets
-// p=1), 20 and 24 (triangles p=4, 5, hexes p=1), 30 (tets p=2), 45 (hexes p=2), 50 (tets
-// p=3), 75 (tets p=4).  launch(RCH, CPW) with integral constants.
+// share of the work, so the block sizes of the element families (hfem_create takes no
+// others) have one that fits: 8-16 (triangles p=1-3, tets p=1), 20 and 24 (triangles p=4,
+// 5, hexes p=1), 30 (tets p=2), 45 (hexes p=2), 50 (tets p=3), 75 (tets p=4).
+// launch(RCH, CPW) with integral constants.
+constexpr int MAX_BLOCK = 80;
+
 template <class F>
 static hipError_t block_shape(int bsz, F launch)
 {
 #define SHAPE(R, C) launch(std::integral_constant<int, R>(), std::integral_constant<int, C>())
-    if (bsz < 1 || bsz > 128) return hipErrorInvalidValue;
+    if (bsz < 1 || bsz > MAX_BLOCK) return hipErrorInvalidValue;
     if (bsz <= 16) SHAPE(1, 4);
     else if (bsz <= 24) SHAPE(1, 6);
     else if (bsz <= 32) SHAPE(1, 8);
     else if (bsz <= 48) SHAPE(1, 12);
     else if (bsz <= 52) SHAPE(1, 13);
-    else if (bsz <= 64) SHAPE(1, 16);
-    else if (bsz <= 80) SHAPE(2, 20);
-    else SHAPE(2, 32);
+    else SHAPE(2, 20);
 #undef SHAPE
     return hipGetLastError();
 }
@@ -1629,17 +1630,16 @@ size_t block_inverse_lds(int bsz)
 {
     return sizeof(double) * (bsz * bsz + 1) / 16 * 16 + 16 + InvShared<double>::bytes(bsz);
 }
-// (no factorisation shape beyond a block size of 80)
-size_t bilu0_factor_lds(int bsz) { return bsz <= 80 ? factor_lds<double>(bsz) : ~(size_t)0 / 2; }
+size_t bilu0_factor_lds(int bsz) { return bsz <= MAX_BLOCK ? factor_lds<double>(bsz) : ~(size_t)0 / 2; }
 
 hipError_t launch_block_inverse(int nrows, int bsz, const int *rowpts, const double *Hg, double *Dinv, int *info,
                                 hipStream_t s)
 {
     const size_t lds = block_inverse_lds(bsz);
-    if (bsz < 1 || bsz > 128) return hipErrorInvalidValue;
+    if (bsz < 1 || bsz > MAX_BLOCK) return hipErrorInvalidValue;
     const int nt = (bsz + 15) / 16;
     auto kernel = nt == 1 ? block_inverse_kernel<1> : nt == 2 ? block_inverse_kernel<2> : nt == 3 ? block_inverse_kernel<3>
-                : nt == 4 ? block_inverse_kernel<4> : nt == 5 ? block_inverse_kernel<5> : block_inverse_kernel<8>;
+                : nt == 4 ? block_inverse_kernel<4> : block_inverse_kernel<5>;
     hipError_t e = set_lds((const void *)kernel, lds);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(kernel, dim3(std::min(nrows, 8192)), dim3(SV_THREADS), lds, s, nrows, bsz, rowpts, Hg, Dinv,
@@ -1647,20 +1647,10 @@ hipError_t launch_block_inverse(int nrows, int bsz, const int *rowpts, const dou
     return hipGetLastError();
 }
 
-// (block sizes above 80 have no factorisation shape: bilu0_factor_lds)
-template <class F>
-static hipError_t factor_shape(int bsz, F launch)
-{
-    if (bsz > 80) return hipErrorInvalidValue;
-    return block_shape(bsz, [&](auto R, auto C) {
-        if constexpr (C() <= 20) launch(R, C);
-    });
-}
-
 hipError_t launch_mdf_weights(int nrows, int bsz, const int *rowpts, const double *Hg, const double *Dinv,
                               double *Cw, hipStream_t s)
 {
-    return factor_shape(bsz, [&](auto, auto C) {
+    return block_shape(bsz, [&](auto, auto C) {
         hipLaunchKernelGGL(mdf_weight_kernel<C()>, dim3(std::min(nrows, 8192)), dim3(SV_THREADS),
                            sizeof(double) * bsz * bsz, s, nrows, bsz, rowpts, Hg, Dinv, Cw);
     });
@@ -1671,7 +1661,7 @@ static hipError_t factor_level(int bsz, const int *rowpts, const int *colind, co
                                int t0, int t1, T *Mg, int *info, hipStream_t s)
 {
     const size_t lds = factor_lds<T>(bsz);
-    return factor_shape(bsz, [&](auto R, auto C) {
+    return block_shape(bsz, [&](auto R, auto C) {
         if (set_lds((const void *)bilu0_factor_kernel<T, R(), C()>, lds) == hipSuccess)
             hipLaunchKernelGGL((bilu0_factor_kernel<T, R(), C()>), dim3(std::min(t1 - t0, 8192)), dim3(SV_THREADS), lds,
                                s, bsz, rowpts, colind, u2o, sch, t0, t1, Mg, info);
@@ -1686,7 +1676,7 @@ static hipError_t factor_syncfree(int bsz, const int *rowpts, const int *colind,
     if (n <= 0 || nwg <= 0) return hipErrorInvalidValue;
     const size_t lds = factor_lds<T>(bsz);
     hipLaunchKernelGGL(factor_reset_kernel, dim3(1), dim3(64), 0, s, sync);
-    return factor_shape(bsz, [&](auto R, auto C) {
+    return block_shape(bsz, [&](auto R, auto C) {
         if (set_lds((const void *)bilu0_factor_syncfree_kernel<T, R(), C()>, lds) == hipSuccess)
             hipLaunchKernelGGL((bilu0_factor_syncfree_kernel<T, R(), C()>), dim3(std::min(n, nwg)), dim3(SV_THREADS),
                                lds, s, bsz, rowpts, colind, u2o, sch, n, Mg, info, flags, sync, sync + 1, spin_limit,
@@ -1728,7 +1718,7 @@ static hipError_t scale_upper(int bsz, int n, const int *rowpts, const int *coli
                               hipStream_t s)
 {
     if (n <= 0) return hipSuccess;
-    return factor_shape(bsz, [&](auto, auto C) {
+    return block_shape(bsz, [&](auto, auto C) {
         hipLaunchKernelGGL((bilu0_scale_upper_kernel<C(), TM>), dim3(std::min(n, 8192)), dim3(SV_THREADS),
                            sizeof(double) * bsz * bsz, s, bsz, n, rowpts, colind, u2o, Mg);
     });
@@ -1818,7 +1808,7 @@ hipError_t launch_bilu0_syncfree(int bsz, const int4 *lrows, const int2 *lnbr, c
 template <typename TM>
 static hipError_t bj(int nrows, int bsz, const TM *Dinv, const double *x, double *y, hipStream_t s)
 {
-    if (bsz > 128) return hipErrorInvalidValue;
+    if (bsz > MAX_BLOCK) return hipErrorInvalidValue;
     const int wpb = SV_THREADS / 64;
     hipLaunchKernelGGL(block_jacobi_kernel<TM>, dim3(std::min((nrows + wpb - 1) / wpb, 8192)), dim3(SV_THREADS), 0,
                        s, nrows, bsz, Dinv, x, y);
