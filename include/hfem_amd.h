@@ -68,7 +68,8 @@ int hfem_set_physics(hfem_ctx *ctx, const double *physicsparam, const double *ui
                      double fc_q, int tdep);
 
 /* Mesh: dgnodes (ne,nd,npv), elcon (ne,nfe,npf), bf (ne,nfe; <0 boundary),
- * t2f (ne,nfe); BSR trace graph rowstart[nf+1], cols[nblocks] (self block first). */
+ * t2f (ne,nfe); BSR trace graph rowstart[nf+1], cols[nblocks] (self block first,
+ * columns below nf). */
 int hfem_set_mesh(hfem_ctx *ctx, const double *dgnodes, const int *elcon, const int *bf, const int *t2f,
                   const int *rowstart, const int *cols, int nblocks);
 
